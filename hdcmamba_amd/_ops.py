@@ -828,6 +828,21 @@ def gemm(x, weight, bias=None, out=None):
     return out
 
 
+def gemm_preferred(x, weight, bias) -> bool:
+    """Whether linear(x, weight, bias) runs on the tiled GEMM (gemm) rather than the library's:
+    bf16 in the layout it takes, K <= 768 and at most 32768 rows, where the library's default
+    solution measured slower (in_proj, N = 4 K + 192: K 768, 32768 rows 264 against 201 us, 8192
+    rows 70 against 55; K 512, 8192 rows 39 against 32; K 256, 16384 rows 34 against 23) -- at
+    K 1024 it is 255 against 318 us, at 131072 rows and K 512 387 against 459.  With recorded
+    library solutions in use (use_tuned_gemms: 162 us at the first shape) the library keeps all."""
+    K = x.shape[-1]
+    rows = x.numel() // K if K else 0
+    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and bias.dtype == torch.bfloat16
+            and 0 < K <= 768 and 0 < rows <= 32768 and K % 8 == 0 and weight.shape[0] % 4 == 0 and weight.shape[1] == K
+            and x.is_contiguous() and weight.is_contiguous() and bias.is_contiguous() and x.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0 and bias.data_ptr() % 8 == 0 and not torch.cuda.tunable.is_enabled())
+
+
 def rowln_gemm(c, weight, residual, eps=1e-5, out=None):
     """residual + LN(c) @ weight^T, LN the row LayerNorm without affine over c's last dim;
     the row statistics and the weight's row sums are computed inside the GEMM.  ``out`` may

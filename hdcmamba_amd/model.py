@@ -242,7 +242,9 @@ class HdcMamba9v3Block(nn.Module):
         ds, H, C = self.d_state, self.num_heads, self.chunk_size
         dtype = x.dtype
         x_conv = fused_norm_conv1d_trainable(x, self.norm, self.conv1d)
-        projs = F.linear(x_conv, self.in_proj.weight.to(dtype), self.in_proj.bias.to(dtype))
+        w_in, b_in = self.in_proj.weight.to(dtype), self.in_proj.bias.to(dtype)
+        # the SSM and slot kernels are constants for autograd, so projs needs no graph either
+        projs = _ops.gemm(x_conv, w_in, b_in) if _ops.gemm_preferred(x_conv, w_in, b_in) else F.linear(x_conv, w_in, b_in)
         combined = torch.empty(B, L, ds + dm, device=x.device, dtype=dtype)
         # The SSM and the slot kernels read projs and write disjoint columns of `combined`,
         # so the SSM may run on a side stream beside some of the slot kernels (ssm_overlap:

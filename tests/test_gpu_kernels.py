@@ -631,7 +631,7 @@ def _block_sums(vals, width):
     """[rows, cols] -> [rows, ceil(cols / width), 2] fp64 (sum, sum of squares) per column block."""
     v = vals.double()
     nb = -(-v.shape[1] // width)
-    out = torch.zeros(v.shape[0], nb, 2, dtype=torch.float64)
+    out = torch.zeros(v.shape[0], nb, 2, dtype=torch.float64, device=v.device)
     for i in range(nb):
         blk = v[:, i * width:(i + 1) * width]
         out[:, i, 0] = blk.sum(1)
@@ -713,6 +713,30 @@ def test_rowln_gemm_stats(dev, M, N, K, mean):
     _ops.rowln_gemm_stats(cd, Wd, ws, st, rd, out=rd)  # out aliasing the residual
     torch.cuda.synchronize()
     assert torch.equal(rd.cpu(), out.cpu())
+
+
+@pytest.mark.parametrize("M,N,K", [
+    # one shape per tile width and edge: 64 (last tiles one row / 8 columns over), 128 (rows and
+    # columns past whole tiles, two and more tiles per CU, K one chunk past a step), 256 (more
+    # than one round, both edges ragged)
+    (65, 72, 64), (449, 520, 136), (2049, 3272, 776), (6000, 1160, 520), (16300, 1032, 1152), (8200, 3264, 768)])
+def test_gemm_tile_widths(dev, M, N, K):
+    """Every tile width of the tiled GEMM with each of its epilogues on one shape, against torch
+    fp32: one bf16 rounding of the result plus fp32 sums of K products of size ~1/sqrt(K) (and of
+    the row statistics, ~1e-3 after the residual)."""
+    _say("gemm tiles", M, N, K)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    c = (1.5 * torch.randn(M, K, generator=g, device=dev) + 0.5).to(torch.bfloat16)
+    W = (torch.randn(N, K, generator=g, device=dev) / K ** 0.5).to(torch.bfloat16)
+    b = (0.1 * torch.randn(N, generator=g, device=dev)).to(torch.bfloat16)
+    r = torch.randn(M, N, generator=g, device=dev).to(torch.bfloat16)
+    st = _block_sums(c, 64).float().transpose(0, 1).contiguous()
+    lin = c.float() @ W.float().t() + b.float()
+    ln = r.float() + torch.nn.functional.layer_norm(c.float(), (K,), eps=1e-5) @ W.float().t()
+    for what, out, ref in (("bias", _ops.gemm(c, W, b), lin), ("rowln", _ops.rowln_gemm(c, W, r), ln),
+                           ("stats", _ops.rowln_gemm_stats(c, W, _ops.row_sums(W), st, r), ln)):
+        err = (out.float() - ref).abs()
+        assert (err <= 2 ** -8 * ref.abs() + 2e-3).all(), f"{what}: max err {err.max().item()}"
 
 
 def test_fused_out_proj_matches_unfused(dev):

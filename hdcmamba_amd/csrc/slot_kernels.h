@@ -261,6 +261,34 @@ struct TileLoader {
   }
 };
 
+// One operand block's rows in 16-byte groups, GPT = TC * HD / E of them over the workgroup's
+// threads (TileLoader for a single block with its own row stride).
+template <typename T, int HD, int TC>
+struct RowLoader {
+  static constexpr int E = Vec<T>::N, GPR = HD / E, GPT = TC * GPR;
+  static constexpr int N = (GPT + kThreads - 1) / kThreads;
+  static constexpr bool EXACT = GPT % kThreads == 0;
+  static __device__ __forceinline__ bool valid(int it, int tid) { return EXACT || tid + kThreads * it < GPT; }
+  // N loads whatever tlen: rows past the tile and idle threads read row 0 (zeroed when staged).
+  static __device__ __forceinline__ void load(uint4* raw, const T* tile_base, int64_t rs, int tlen, int tid) {
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      const int idx = tid + kThreads * it, r = idx / GPR;
+      const bool ok = valid(it, tid) && r < tlen;
+      raw[it] = ldg16(tile_base + (ok ? (int64_t)r * rs : 0) + (valid(it, tid) ? idx % GPR : 0) * E);
+    }
+  }
+  // as stored, row-major with pitch P; rows past the tile zero
+  static __device__ __forceinline__ void stage(const uint4* raw, T* dst, int P, int tlen, int tid) {
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      if (!valid(it, tid)) continue;
+      const int idx = tid + kThreads * it, r = idx / GPR;
+      *reinterpret_cast<uint4*>(dst + r * P + idx % GPR * E) = r < tlen ? raw[it] : make_uint4(0, 0, 0, 0);
+    }
+  }
+};
+
 // Write a loaded tile to LDS.  q: phi(q) row-major.  k: phi(k) row-major (unless
 // STATE_ONLY) and (phi(k)*gamma^(tlen-1-i))^T.  v: v^T.  Rows >= tlen are zero.  Without
 // PHI the feature map is the identity (q and k staged as they are).
@@ -736,13 +764,15 @@ __global__ __launch_bounds__(kThreads, HD > 64 ? 1 : (HAS_W ? 2 : kGateWavesPerE
 }
 
 // Per (segment, head, batch): U_s = sum_{j in segment} gamma^(end-1-j) k~_j^T v_j, with k~
-// from phi(k) (PHI) or k itself.  k starts at column k_col of each row, v v_off columns later.
-template <typename T, int HD, int TC, bool PHI>
+// from phi(k) (PHI) or k itself.  k starts at column k_col of each row, v v_off columns later, or
+// (SPLIT) in rows of its own at v_base, row stride v_rs.
+template <typename T, int HD, int TC, bool PHI, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads, HD > 64 ? 2 : 4) void slot_state_kernel(const T* __restrict__ projs,
                                                               int64_t prs, int k_col, int v_off,
                                                               int L, const T* __restrict__ gamma,
                                                               int seg_rows, int nseg,
-                                                              float* __restrict__ U) {
+                                                              float* __restrict__ U,
+                                                              const T* __restrict__ v_base, int64_t v_rs) {
   using LD = Lds<T, HD, TC>;
   using TL = TileLoader<T, HD, TC, 1, 2>;
   __shared__ __attribute__((aligned(16))) T sm[LD::stTotal];
@@ -770,19 +800,29 @@ __global__ __launch_bounds__(kThreads, HD > 64 ? 2 : 4) void slot_state_kernel(c
   // re-read the current tile, and the loop body always runs both steps (tlen = 0 makes a
   // step a no-op: zero tile, gamma^0 = 1), so every path issues the same loads in the same
   // order and the compiler's memory-counter waits stay exact.
-  const TL loader(prs, {0, v_off}, tid);
+  const TL kv_loader(prs, {0, v_off}, tid);
   uint4 raw0[TL::NL], raw1[TL::NL];
   const T* tbase = colbase + rowbase * prs;
+  const T* vbase = SPLIT ? v_base + h * HD + rowbase * v_rs : nullptr;
+  auto load = [&](uint4 (&raw)[TL::NL], int p) {
+    const int tlen = min(TC, p_end - p);
+    if constexpr (SPLIT) {
+      using RL = RowLoader<T, HD, TC>;
+      RL::load(raw, tbase + (int64_t)p * prs, prs, tlen, tid);
+      RL::load(raw + RL::N, vbase + (int64_t)p * v_rs, v_rs, tlen, tid);
+    } else {
+      kv_loader.load(raw, tbase + (int64_t)p * prs, tlen);
+    }
+  };
   // U_s is a decayed sum over the segment's rows, so the tiles need not follow chunks
   const int p1 = p_begin + TC < p_end ? p_begin + TC : p_begin;
-  loader.load(raw0, tbase + (int64_t)p_begin * prs, min(TC, p_end - p_begin));
-  loader.load(raw1, tbase + (int64_t)p1 * prs, min(TC, p_end - p1));
+  load(raw0, p_begin);
+  load(raw1, p1);
 
   auto step = [&](uint4 (&raw)[TL::NL], int p, int tlen) {
     __syncthreads();
     stage_tile<T, HD, TC, 1, 2, true, PHI>(raw, sm, tlen, lg2, tid);
-    const int pn = p + 2 * TC < p_end ? p + 2 * TC : p;
-    loader.load(raw, tbase + (int64_t)pn * prs, min(TC, p_end - pn));
+    load(raw, p + 2 * TC < p_end ? p + 2 * TC : p);
     __syncthreads();
     const float gt = fexp2((float)tlen * lg2);
 #pragma unroll
@@ -945,7 +985,7 @@ int launch_state(const void* base, int64_t prs, int64_t k_col, int64_t v_off, co
   if (pl.nseg > 1) {
     HDCM_LAUNCH((slot_state_kernel<T, HD, TC, PHI>), dim3((unsigned)H, pl.nseg - 1, (unsigned)B),
                        dim3(kThreads), 0, s, (const T*)base, prs, (int)k_col, (int)v_off, (int)L,
-                       (const T*)gamma, pl.seg_rows, pl.nseg, U);
+                       (const T*)gamma, pl.seg_rows, pl.nseg, U, (const T*)nullptr, (int64_t)0);
     const int st = hdcm_launch_status();
     if (st) return st;
   }

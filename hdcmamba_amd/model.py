@@ -126,10 +126,9 @@ class SlotSsmMixerFunction(torch.autograd.Function):
     the ``combined`` rows [y_ssm | gated slot output] of the forward (model.py:345-380).
     The backward (no counterpart in the reference, whose kernels have no autograd) returns
     the gradients of projs, A_log and the GroupNorm parameters; gamma (the slot decay, a
-    buffer refreshed from decay_log) is treated as a constant.  Slot part: y recomputed by
-    the plain recurrence, the GroupNorm/gate backward, then three passes of the recurrence
-    for d phi(q), d v and d phi(k) (the last two backwards in time) and the phi' chain;
-    SSM part: the adjoint scan from the forward's y.
+    buffer refreshed from decay_log) is treated as a constant.  Slot part: two passes over the
+    sequence (hdcm_slot_grad), the first from the segment states that the forward left; SSM
+    part: the adjoint scan from the forward's y.
     """
 
     @staticmethod
@@ -140,32 +139,21 @@ class SlotSsmMixerFunction(torch.autograd.Function):
         ws = _ops.slot_workspace(projs, dm, H, C)
         _ops.slot_state(projs, 3 * ds, gamma, dm, H, C, ws)
         _ops.slot_gate(projs, 3 * ds, gamma, gn_w, gn_b, 1e-5, ws, combined, ds, dm, H, C)
-        ctx.save_for_backward(projs, A_log, gamma, gn_w, gn_b, combined)
+        ctx.save_for_backward(projs, A_log, gamma, gn_w, gn_b, combined, ws)
         ctx.dims = (ds, dm, H, C)
+        ctx.seg_tiles = _ops.option_value("slot_seg_tiles")
         return combined
 
     @staticmethod
     def backward(ctx, dcomb):
-        projs, A_log, gamma, gn_w, gn_b, combined = ctx.saved_tensors
+        projs, A_log, gamma, gn_w, gn_b, combined, ws = ctx.saved_tensors
         ds, dm, H, C = ctx.dims
-        B, L, _ = projs.shape
         dcomb = dcomb.to(projs.dtype).contiguous()
-        q_col, g_col = 3 * ds, 3 * ds + 3 * dm
         dprojs = torch.empty_like(projs)
-        ws = _ops.slot_workspace(projs, dm, H, C)
-        y = torch.empty(B, L, dm, device=projs.device, dtype=projs.dtype)
-        _ops.slot_attend(projs, q_col, q_col + dm, q_col + 2 * dm, gamma, dm, H, C, True, y, 0, ws=ws)
-        z = torch.empty(B, L, 4 * dm, device=projs.device, dtype=projs.dtype)  # [dy | v | phi(k) | phi(q)]
-        dgw, dgb = _ops.gnorm_gate_bwd(y, projs[..., g_col:], gn_w, gn_b, 1e-5, dcomb[..., ds:], H,
-                                       z[..., :dm], dprojs[..., g_col:])
-        _ops.slot_phi_prep(projs, q_col, dm, z)
-        # d q = d phi(q) * phi'(q) and d k likewise: the passes multiply by phi' of the
-        # projections (chain) as they store
-        _ops.slot_attend(z, 0, dm, 2 * dm, gamma, dm, H, C, False, dprojs, q_col, ws=ws, chain=projs)  # d q
-        _ops.slot_attend(z, 2 * dm, 3 * dm, 0, gamma, dm, H, C, False, dprojs, q_col + 2 * dm, reverse=True,
-                         ws=ws)  # d v
-        _ops.slot_attend(z, dm, 0, 3 * dm, gamma, dm, H, C, False, dprojs, q_col + dm, reverse=True,
-                         ws=ws, chain=projs)  # d k
+        if ctx.seg_tiles != _ops.option_value("slot_seg_tiles"):  # the states were cut into other segments
+            ws = _ops.slot_workspace(projs, dm, H, C)
+            _ops.slot_state(projs, 3 * ds, gamma, dm, H, C, ws)
+        dgw, dgb = _ops.slot_grad(projs, 3 * ds, gamma, gn_w, gn_b, 1e-5, ws, dcomb[..., ds:], dprojs, dm, H, C)
         dA = _ops.ssm_bwd(projs, A_log, ds, combined[..., :ds], dcomb[..., :ds], dprojs)
         return (dprojs, dA.to(A_log.dtype), None, dgw.to(gn_w.dtype), dgb.to(gn_b.dtype), None, None, None, None)
 

@@ -287,6 +287,22 @@ int hdcm_gnorm_gate_bwd(const void* y, int64_t y_row_stride, const void* gate, i
                         int64_t rows, int64_t dm, int64_t H, int dtype, void* stream);
 
 /*
+ * Gradient of hdcm_slot_state_fwd + hdcm_slot_gate_fwd (gamma constant) in two passes: writes the
+ * q, k, v and gate column blocks of dprojs (4 dm columns from q_col on, activation dtype) and
+ * d gn_w, d gn_b (fp32 [dm], summed in a fixed order) from projs, dout [B*L, dm] and ws_fwd, the
+ * workspace as the two forward calls left it (same B, L, dm, H, C, dtype, and the same
+ * HDCM_OPT_SLOT_SEG_TILES).  dprojs may not overlap projs or dout.  Rows 16-byte aligned.
+ * ws: hdcm_slot_grad_workspace_bytes bytes.  hd a multiple of 16 up to 128.
+ * No reference counterpart (model.py:236-295 has no backward).
+ */
+size_t hdcm_slot_grad_workspace_bytes(int64_t B, int64_t L, int64_t dm, int64_t H, int64_t C, int dtype);
+int hdcm_slot_grad(const void* projs, int64_t proj_row_stride, int64_t q_col, const void* gamma, const void* gn_w,
+                   const void* gn_b, float gn_eps, const void* ws_fwd, size_t ws_fwd_bytes, const void* dout,
+                   int64_t dout_row_stride, void* dprojs, int64_t dprojs_row_stride, float* dgn_w, float* dgn_b,
+                   void* ws, size_t ws_bytes, int64_t B, int64_t L, int64_t dm, int64_t H, int64_t C, int dtype,
+                   void* stream);
+
+/*
  * Operands of the slot recurrence's gradient passes.  hdcm_slot_phi_prep writes, per row,
  * v, phi(k) and phi(q) (rounded to the dtype) into column blocks [dm, 2dm), [2dm, 3dm) and
  * [3dm, 4dm) of z (q, k, v at columns q_col, +dm, +2dm of projs).  hdcm_slot_phi_chain turns

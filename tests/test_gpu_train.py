@@ -268,3 +268,57 @@ def test_differentiable_mixer_block(dev, dtype, L, dm, H, C):
     _say(f"  x: {err:.2e}")
     assert err <= lim
     assert params["decay_log"].grad is None
+
+
+@pytest.mark.parametrize("dtype,B,L,H,hd,ds,C,seg", [
+    (torch.bfloat16, 2, 192, 2, 64, 16, 64, 0),      # whole tiles, one segment
+    (torch.bfloat16, 1, 1024, 2, 64, 8, 256, 2),     # chunk of four tiles (carried W), 256-row segments
+    (torch.bfloat16, 2, 320, 3, 32, 8, 16, 1),       # four chunks per tile, one tile per segment
+    (torch.bfloat16, 1, 300, 2, 48, 8, 100, 1),      # chunk-confined tiles of 64 and 36 rows, odd tile count
+    (torch.bfloat16, 2, 60, 1, 16, 8, 20, 0),        # one short tile, smallest head
+    (torch.bfloat16, 1, 192, 2, 96, 8, 64, 1), (torch.bfloat16, 1, 256, 2, 128, 8, 128, 1),
+    (torch.bfloat16, 1, 70, 1, 112, 8, 70, 0), (torch.bfloat16, 1, 128, 1, 80, 8, 32, 1),
+    (torch.float32, 2, 192, 2, 64, 4, 64, 1), (torch.float32, 1, 256, 2, 32, 4, 32, 2),
+    (torch.float32, 1, 120, 2, 48, 4, 40, 1), (torch.float32, 2, 64, 1, 16, 4, 8, 1),
+    (torch.float32, 1, 192, 1, 128, 4, 96, 1), (torch.float32, 1, 96, 1, 112, 4, 96, 0),
+    (torch.float32, 1, 64, 2, 96, 4, 16, 0), (torch.float32, 1, 80, 1, 80, 4, 80, 0),
+])
+def test_slot_gradient_passes(dev, dtype, B, L, H, hd, ds, C, seg):
+    """SlotSsmMixerFunction's gradients of q, k, v, the gate and the GroupNorm against autograd
+    through the oracle's slot recurrence and GroupNorm on the same rounded inputs: every tile form
+    (whole, several chunks to a tile, several tiles to a chunk, chunk-confined), odd and even head
+    tile counts, one and many segments.  Bounds as for the differentiable block (fp32 sums in
+    another order; bf16 operands rounded once per product, ~2^-8 of the largest value)."""
+    from hdcmamba_amd import _ops
+    from hdcmamba_amd.model import SlotSsmMixerFunction
+
+    dm = H * hd
+    _say("slot gradient", dtype, B, L, H, hd, C, seg)
+    g = torch.Generator().manual_seed(L + hd + C)
+    projs = torch.randn(B, L, 3 * ds + 4 * dm, generator=g).to(dtype)
+    gamma = (0.9 + 0.09 * torch.rand(H, generator=g)).to(dtype)
+    w = (1 + 0.2 * torch.randn(dm, generator=g)).to(dtype)
+    b = (0.1 * torch.randn(dm, generator=g)).to(dtype)
+    do = torch.randn(B, L, ds + dm, generator=g).to(dtype)
+    A_log = torch.log(torch.linspace(0.5, 2.0, ds)).to(dtype)
+    pr, wr, br = (t.double().clone().requires_grad_(True) for t in (projs, w, b))
+    q, k, v, gate = (pr[..., 3 * ds + i * dm:3 * ds + (i + 1) * dm].reshape(B, L, H, hd) for i in range(4))
+    t = torch.arange(L)
+    e = t[:, None] - t[None] - (t[:, None] // C != t[None] // C).long()
+    wts = torch.where(t[:, None] >= t[None], gamma.double()[:, None, None] ** e.clamp(min=0), 0.0)
+    f = lambda z: torch.where(z > 0, z + 1, torch.exp(z.clamp(max=0)))  # noqa: E731
+    y = torch.einsum("bthd,bshd->bhts", f(q), f(k)) * wts
+    y = torch.einsum("bhts,bshd->bthd", y, v)
+    yn = torch.nn.functional.group_norm(y.reshape(B * L, dm), H, wr, br, 1e-5).view(B, L, dm)
+    (yn * torch.sigmoid(gate.reshape(B, L, dm)) * do[..., ds:].double()).sum().backward()
+    leaves = [x.to(dev).requires_grad_(True) for x in (projs, A_log, w, b)]
+    with _ops.option("slot_seg_tiles", seg):
+        out = SlotSsmMixerFunction.apply(leaves[0], leaves[1], gamma.to(dev), leaves[2], leaves[3], ds, dm, H, C)
+        got = torch.autograd.grad(out, leaves, do.to(dev))
+    lim = 1e-4 if dtype == torch.float32 else 2e-2
+    blocks = [(n, got[0][..., 3 * ds + i * dm:3 * ds + (i + 1) * dm], pr.grad[..., 3 * ds + i * dm:3 * ds + (i + 1) * dm])
+              for i, n in enumerate(("d q", "d k", "d v", "d gate"))]
+    for name, x, ref in [*blocks, ("d gn_w", got[2], wr.grad), ("d gn_b", got[3], br.grad)]:
+        err = max_rel(x, ref)
+        _say(f"  {name}: {err:.2e}")
+        assert err <= lim, (name, err)

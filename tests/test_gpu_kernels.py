@@ -7,7 +7,7 @@ import torch
 
 import oracle
 from hdcmamba_amd import _ops
-from cfgs import assert_close, slot_inputs, ssm_inputs
+from cfgs import assert_close, max_rel, slot_inputs, ssm_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -47,6 +47,36 @@ def test_norm_conv_wide_rows_bf16(dev, D, L):
 def test_norm_conv_backward_wide_bf16(dev, D, L):
     """bf16 rows up to the forward's 6144 columns through the shared-row backward kernel."""
     test_norm_conv_backward(dev, torch.bfloat16, 1, L, D)
+
+
+@pytest.mark.parametrize("dtype,B,L,D", [
+    # one, two and four waves per row; a row of one lane; runs of 16 rows ending inside and at a
+    # sequence's end, an odd number of them (the last workgroup's second slice has none), one row,
+    # runs longer than 16 rows (more than 2048 / waves-per-row of them), two and three groups per lane
+    (torch.bfloat16, 3, 17, 8), (torch.bfloat16, 1, 1, 512), (torch.bfloat16, 3, 16, 520), (torch.bfloat16, 1, 33, 1024),
+    (torch.bfloat16, 2, 5, 1032), (torch.bfloat16, 1, 9001, 1032), (torch.bfloat16, 1, 20, 2056), (torch.bfloat16, 1, 19, 4104),
+    (torch.float32, 3, 17, 4), (torch.float32, 1, 2, 260), (torch.float32, 5, 16, 516), (torch.float32, 2, 18, 1028),
+    (torch.float32, 1, 9001, 1536), (torch.float32, 1, 17, 2052)])
+def test_norm_conv_backward_runs(dev, dtype, B, L, D):
+    """hdcm_norm_conv_bwd's run and row splits against autograd in fp64 on the same rounded inputs:
+    fp32 sums over B L rows (1e-4 of the largest gradient), one bf16 rounding of dx."""
+    _say("norm_conv bwd runs", dtype, B, L, D)
+    g = torch.Generator(device=dev).manual_seed(B + L + D)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    x, go = (1.5 * r(B, L, D) + 0.5).to(dtype), r(B, L, D).to(dtype)
+    w, b, cw = (1 + 0.2 * r(D)).to(dtype), (0.3 * r(D)).to(dtype), (0.3 * r(D, 4)).to(dtype)
+    xr, wr, br, cr = (t.double().requires_grad_() for t in (x, w, b, cw))
+    u = torch.nn.functional.layer_norm(xr, (D,), wr, br, 1e-5)
+    u = torch.cat([br.expand(B, 3, D), u], 1)
+    out = sum(u[:, k:k + L] * cr[:, k] for k in range(4))
+    ref = torch.autograd.grad(out, [xr, wr, br, cr], go.double())
+    got = _ops.norm_conv_bwd(go, x, w, b, cw, 1e-5)
+    if D > 8:  # (a LayerNorm over 4 or 8 columns amplifies: dx is compared on the wider rows)
+        err = (got[0].double() - ref[0]).abs() - (2 ** -8 if dtype == torch.bfloat16 else 1e-4) * ref[0].abs()
+        assert err.max() <= 1e-4 * ref[0].abs().max(), f"dx {err.max().item()}"
+    for name, a, e in (("ln_w", got[1], ref[1]), ("ln_b", got[2], ref[2]), ("conv_w", got[3], ref[3]),
+                       ("conv_b", got[4], go.double().sum((0, 1)))):
+        assert max_rel(a, e) <= 1e-4, (name, max_rel(a, e))
 
 
 def test_norm_conv_batch_strided(dev):

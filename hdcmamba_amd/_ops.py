@@ -8,6 +8,7 @@ or fallback path: a missing library or a CPU tensor raises.
 from __future__ import annotations
 
 import ctypes
+import importlib
 from ctypes import c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
@@ -46,6 +47,11 @@ _PROTOS = {
                                    c_void_p]),
     "hdcm_slot_phi_chain": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int,
                                     c_void_p]),
+    "hdcm_pad_rows_fwd": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int,
+                                  c_void_p]),
+    "hdcm_gamma_fwd": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
+    "hdcm_stream_after": (c_int, [c_void_p, c_void_p, c_int]),
+    "hdcm_gemm_preferred": (c_int, [c_int64, c_int64, c_int64, c_int]),
     "hdcm_slot_grad_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int]),
     "hdcm_slot_grad": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_size_t,
                                c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_size_t, c_int64,
@@ -115,6 +121,22 @@ def lib() -> ctypes.CDLL:
             raise RuntimeError(f"{LIB_PATH.name} ABI {h.hdcm_abi_version()} != expected {ABI_VERSION}")
         _lib = h
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The native host path (csrc/native.cpp), imported once."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            _native = importlib.import_module("hdcmamba_amd._native")
+        except ImportError as e:
+            raise RuntimeError("hdcmamba_amd/_native.so is not built or does not load; run `python -m hdcmamba_amd.build` "
+                               f"({e})") from e
+    return _native
 
 
 class HdcmError(RuntimeError):
@@ -385,6 +407,25 @@ def _ssm_workspace(device, nbytes):
         ws = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
         _ssm_ws[key] = ws
     return ws
+
+
+def native_streams(t, L, d_state, overlap):
+    """(main stream, side stream, overlap code, the scan's workspace) for the native host path on t
+    [B, ..]'s device.  ``overlap`` as HdcMamba9v3Block.ssm_overlap; "auto" runs the scan on the
+    current stream, on that stream's workspace -- in a recorded graph, whose capture stream has
+    none, on the side stream's, which every eager call provides for."""
+    main = torch.cuda.current_stream(t.device)
+    nbytes = lib().hdcm_ssm_workspace_bytes(t.shape[0], L, d_state)
+    side = side_stream(t.device)
+    ws = _ssm_ws.get((side.device.index, side.cuda_stream))
+    if ws is None or ws.numel() < nbytes:
+        with torch.cuda.stream(side):
+            ws = _ssm_workspace(t.device, nbytes)
+    if overlap == "auto":
+        if not torch.cuda.is_current_stream_capturing():
+            ws = _ssm_workspace(t.device, nbytes)
+        return main.cuda_stream, main.cuda_stream, native().MAIN, ws
+    return main.cuda_stream, side.cuda_stream, native().OVERLAP[overlap], ws
 
 
 def _stats_arg(row_stats, part, rows, nparts):
@@ -861,17 +902,15 @@ def gemm(x, weight, bias=None, out=None):
 
 def gemm_preferred(x, weight, bias) -> bool:
     """Whether linear(x, weight, bias) runs on the tiled GEMM (gemm) rather than the library's:
-    bf16 in the layout it takes, K <= 768 and at most 32768 rows, where the library's default
-    solution measured slower (in_proj, N = 4 K + 192: K 768, 32768 rows 264 against 201 us, 8192
-    rows 70 against 55; K 512, 8192 rows 39 against 32; K 256, 16384 rows 34 against 23) -- at
-    K 1024 it is 255 against 318 us, at 131072 rows and K 512 387 against 459.  With recorded
-    library solutions in use (use_tuned_gemms: 162 us at the first shape) the library keeps all."""
+    bf16 in the layout it takes at the sizes of hdcm_gemm_preferred.  With recorded library
+    solutions in use (use_tuned_gemms: in_proj at 32768 rows of d_model 768 162 us, the tiled
+    GEMM 201, the library's default 264) the library keeps all."""
     K = x.shape[-1]
-    rows = x.numel() // K if K else 0
     return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and bias.dtype == torch.bfloat16
-            and 0 < K <= 768 and 0 < rows <= 32768 and K % 8 == 0 and weight.shape[0] % 4 == 0 and weight.shape[1] == K
-            and x.is_contiguous() and weight.is_contiguous() and bias.is_contiguous() and x.data_ptr() % 16 == 0
-            and weight.data_ptr() % 16 == 0 and bias.data_ptr() % 8 == 0 and not torch.cuda.tunable.is_enabled())
+            and bool(lib().hdcm_gemm_preferred(x.numel() // K if K else 0, weight.shape[0], K, HDCM_BF16))
+            and weight.shape[1] == K and x.is_contiguous() and weight.is_contiguous() and bias.is_contiguous()
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and bias.data_ptr() % 8 == 0
+            and not torch.cuda.tunable.is_enabled())
 
 
 def rowln_gemm(c, weight, residual, eps=1e-5, out=None):

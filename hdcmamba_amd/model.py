@@ -66,15 +66,16 @@ class FusedNormConv1dFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, norm_weight, norm_bias, conv_weight, conv_bias, eps):
         ctx.save_for_backward(x, norm_weight, norm_bias, conv_weight)
-        ctx.eps = eps
-        return _ops.norm_conv(x, norm_weight, norm_bias, conv_weight, conv_bias, eps)
+        ctx.eps = float(eps)
+        if _ops.timer.active:
+            return _ops.norm_conv(x, norm_weight, norm_bias, conv_weight, conv_bias, eps)
+        return _ops.native().norm_conv_forward(x, norm_weight, norm_bias, conv_weight, conv_bias, ctx.eps, _ops._stream(x))
 
     @staticmethod
     def backward(ctx, grad_output):
         x, norm_weight, norm_bias, conv_weight = ctx.saved_tensors
-        dx, dnw, dnb, dcw, dcb = _ops.norm_conv_bwd(grad_output, x, norm_weight, norm_bias, conv_weight, ctx.eps)
-        return (dx, dnw.to(x.dtype), dnb.to(x.dtype), dcw.to(x.dtype).view_as(conv_weight), dcb.to(x.dtype),
-                None)
+        return (*_ops.native().norm_conv_backward(grad_output, x, norm_weight, norm_bias, conv_weight, ctx.eps,
+                                                  _ops._stream(x)), None)
 
 
 def fused_norm_conv1d_trainable(x, norm_layer, conv_layer):
@@ -133,12 +134,9 @@ class SlotSsmMixerFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, projs, A_log, gamma, gn_w, gn_b, ds, dm, H, C):
-        B, L, _ = projs.shape
-        combined = torch.empty(B, L, ds + dm, device=projs.device, dtype=projs.dtype)
-        _ops.ssm(projs, A_log, ds, combined[..., :ds])
-        ws = _ops.slot_workspace(projs, dm, H, C)
-        _ops.slot_state(projs, 3 * ds, gamma, dm, H, C, ws)
-        _ops.slot_gate(projs, 3 * ds, gamma, gn_w, gn_b, 1e-5, ws, combined, ds, dm, H, C)
+        _ops._on_gpu(projs)
+        streams = _ops.native_streams(projs, projs.shape[1], ds, "auto")
+        combined, ws = _ops.native().mixer_forward(projs, A_log, gamma, gn_w, gn_b, (ds, H, C), streams)
         ctx.save_for_backward(projs, A_log, gamma, gn_w, gn_b, combined, ws)
         ctx.dims = (ds, dm, H, C)
         ctx.seg_tiles = _ops.option_value("slot_seg_tiles")
@@ -148,14 +146,59 @@ class SlotSsmMixerFunction(torch.autograd.Function):
     def backward(ctx, dcomb):
         projs, A_log, gamma, gn_w, gn_b, combined, ws = ctx.saved_tensors
         ds, dm, H, C = ctx.dims
-        dcomb = dcomb.to(projs.dtype).contiguous()
-        dprojs = torch.empty_like(projs)
         if ctx.seg_tiles != _ops.option_value("slot_seg_tiles"):  # the states were cut into other segments
             ws = _ops.slot_workspace(projs, dm, H, C)
             _ops.slot_state(projs, 3 * ds, gamma, dm, H, C, ws)
-        dgw, dgb = _ops.slot_grad(projs, 3 * ds, gamma, gn_w, gn_b, 1e-5, ws, dcomb[..., ds:], dprojs, dm, H, C)
-        dA = _ops.ssm_bwd(projs, A_log, ds, combined[..., :ds], dcomb[..., :ds], dprojs)
-        return (dprojs, dA.to(A_log.dtype), None, dgw.to(gn_w.dtype), dgb.to(gn_b.dtype), None, None, None, None)
+        dprojs, dA, dgw, dgb = _ops.native().mixer_backward(dcomb, projs, A_log, gamma, gn_w, gn_b, combined, ws,
+                                                            (ds, H, C), _ops._stream(projs))
+        return dprojs, dA, None, dgw, dgb, None, None, None, None
+
+
+class BlockTrainFunction(torch.autograd.Function):
+    """One block's training forward and its backward as two native calls: the forward keeps the
+    block and its input only and the backward recomputes the body from the block's parameters of
+    that moment, as the reference's checkpoint does (model.py:391-392).
+
+    ``apply(block, x, pad, *params)`` on the unpadded x [B,L,dm], params those of
+    ``block._grad_params()``.  A backward that is itself to be differentiated
+    (create_graph) runs through the block's Python composition instead.
+    """
+
+    @staticmethod
+    def forward(ctx, block, x, pad, *params):
+        ctx.block, ctx.x, ctx.pad, ctx.mixer = block, x, pad, block.differentiable_mixer
+        ctx.autocast = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+        return block._native_padded(x, pad)
+
+    @staticmethod
+    def backward(ctx, dy):
+        block, x, pad = ctx.block, ctx.x, ctx.pad
+        need = ctx.needs_input_grad
+        params = block._grad_params(ctx.mixer)
+        if torch.is_grad_enabled():
+            with torch.enable_grad(), torch.amp.autocast("cuda", dtype=ctx.autocast[1], enabled=ctx.autocast[0]):
+                y = block._inner_forward(F.pad(x, (0, 0, pad, 0)).contiguous())[:, pad:, :]
+            wanted = [t for t, n in zip((x, *params), (need[1], *need[3:])) if n]
+            grads = iter(torch.autograd.grad(y, wanted, dy, create_graph=True, allow_unused=True))
+            dx = next(grads) if need[1] else None
+            return (None, dx, None, *(next(grads) if n else None for n in need[3:]))
+        native = _ops.native()
+        dt, stream = x.dtype, _ops._stream(x)
+        dyp = dy.to(dt)
+        if pad:
+            x, dyp = native.pad_rows(x, pad, stream), native.pad_rows(dyp, pad, stream)
+        else:
+            x, dyp = x.contiguous(), dyp.contiguous()
+        if ctx.mixer:
+            mask = [need[1], *need[3:10], False, *need[10:]]
+        else:
+            mask = [need[1], *[False] * 10, need[3]]
+        g = native.block_backward(x, dyp, block._params(), block.norm.eps, (block.d_state, block.num_heads, block.chunk_size),
+                                  block._native_streams(x), ctx.mixer, torch.cuda.tunable.is_enabled(), mask)
+        dx = g[0][:, pad:, :] if g[0] is not None and pad else g[0]
+        if ctx.mixer:
+            return (None, dx, None, *g[1:8], *g[9:])
+        return None, dx, None, g[11]
 
 
 class HdcMamba9v3Block(nn.Module):
@@ -176,12 +219,14 @@ class HdcMamba9v3Block(nn.Module):
     ``_fused_out``); otherwise as a row LayerNorm kernel and addmm.
     """
 
-    # where the SSM's launch overlaps the slot kernels (see _mixer): "auto" runs it in sequence
-    # while a HIP graph is being recorded and beside the slot pre-pass and scan otherwise.
-    # Measured at the 24-layer d_model=1024 L=32768 forward: recorded graph 14.46 ms per
-    # forward in sequence against 14.59 overlapped (with no launch gaps to fill, the scan's
-    # workgroups only slow the pre-pass: 25 + 55 us against 24 + 28 us); eager forwards 15.14
-    # overlapped against 15.65 in sequence.
+    # where the SSM's launch overlaps the slot kernels: "none" = a side stream joined before them,
+    # "state" = beside the state pre-pass and scan, "after_state" = beside the scan and the gate
+    # pass, "gate" = beside all three, "auto" = the current stream, before them.  The fork and join
+    # of two streams cost more than the overlap gains once the host keeps the GPU busy: B=1
+    # L=32768 d_model 1024 501-507 us per block with "auto" against 512-517 with "state", B=2 L=3001
+    # d_model 768 125 against 136 us; in a recorded 24-layer forward the overlap lost as well (14.46
+    # ms in sequence, 14.59 overlapped).  (The Python composition, whose launches are the slower
+    # side, keeps "state" for "auto" outside graph capture.)
     ssm_overlap = "auto"
     # decode step: the LayerNorm + conv of the token and in_proj as one launch
     # (hdcm_norm_conv_in_proj_step_fwd: in_proj's weight stream starts while the conv rows are
@@ -311,6 +356,48 @@ class HdcMamba9v3Block(nn.Module):
         _ops.gnorm_gate(y1, y2, projs[..., q_col + 3 * dm:], self.group_norm.weight, self.group_norm.bias, 1e-5, H,
                         combined[..., ds:], row_stats=row_stats, stats_part=_ops.ssm_stats_parts(ds))
 
+    # ------------------------------------------------------------------ native host path
+    def _native_ok(self, x):
+        """Whether the native host path (csrc/native.cpp) takes x: everything but empty inputs, heads
+        wider than the fused slot kernels', launches being timed one by one, and autocast to
+        another dtype; the Python composition below takes the rest, with the same kernels."""
+        return (x.dtype in _ops._DTYPES and self.head_dim <= _ops.SLOT_MAX_HEAD_DIM and x.numel() > 0
+                and not _ops.timer.active and self.ssm_overlap in ("auto", "none", "state", "gate", "after_state")
+                and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype))
+
+    def _params(self):
+        """The parameters in the order the native host path takes them."""
+        return [self.norm.weight, self.norm.bias, self.conv1d.weight, self.conv1d.bias, self.in_proj.weight,
+                self.in_proj.bias, self.A_log, self.gamma_buf, self.group_norm.weight, self.group_norm.bias,
+                self.out_proj.weight]
+
+    def _grad_params(self, mixer=None):
+        """Those that receive a gradient (``mixer``: with the differentiable mixer)."""
+        if not (self.differentiable_mixer if mixer is None else mixer):
+            return [self.out_proj.weight]
+        p = self._params()
+        return p[:7] + p[8:]  # gamma_buf is a constant
+
+    def _native_streams(self, x):
+        return _ops.native_streams(x, x.shape[1], self.d_state, self.ssm_overlap)
+
+    def _native_forward(self, x, state=None, out=None):
+        """The block body on chunk-aligned contiguous x without autograd (_inner_forward)."""
+        w = self.out_proj.weight
+        fused = self._fused_out(x)
+        sums = self._out_weight_sums(w.to(x.dtype)) if fused and _ops.rowln_stats_ok(x, self.d_model) else None
+        return _ops.native().block_forward(
+            x, self._params(), self.norm.eps, (self.d_state, self.num_heads, self.chunk_size), self._native_streams(x),
+            out, fused, sums, torch.cuda.tunable.is_enabled(), None if state is None else state.h,
+            None if state is None else state.S_prev)
+
+    def _native_padded(self, x, pad):
+        """_native_forward on x [B,L,dm] with ``pad`` zero rows in front, which the output leaves out."""
+        if not pad:
+            return self._native_forward(x.contiguous())
+        xp = _ops.native().pad_rows(x, pad, _ops._stream(x))
+        return self._native_forward(xp, out=xp)[:, pad:, :]
+
     def _fused_out(self, x):
         """Whether out_proj runs as the GEMM with the LayerNorm folded in (bf16, no autograd).
         Measured: it pays on the decode step (<= 16 rows: the weight-streaming kernels) and
@@ -385,6 +472,8 @@ class HdcMamba9v3Block(nn.Module):
     def _inner_forward(self, x, state=None):
         """Block body on a chunk-aligned [B,L,dm] input; returns x + out_proj(LN(combined))."""
         B, L, dm = x.shape
+        if not torch.is_grad_enabled() and self._native_ok(x):
+            return self._native_forward(x, state)
         if self._fused_out(x):
             return self._fused_mixer_out(x, state)
         if self.differentiable_mixer and state is None and torch.is_grad_enabled():
@@ -400,8 +489,8 @@ class HdcMamba9v3Block(nn.Module):
         """In-place variant for a model-owned residual stream r [B,L,dm] (chunk-aligned):
         r += out_proj(LN(combined)), with the GEMM accumulating straight into r."""
         B, L, dm = r.shape
-        if state is not None:
-            self._capture_conv(r, state)
+        if not torch.is_grad_enabled() and self._native_ok(r) and r.is_contiguous():
+            return self._native_forward(r, state, out=r)
         if self._fused_out(r):
             self._fused_mixer_out(r, state, out=r)
             return r
@@ -418,13 +507,19 @@ class HdcMamba9v3Block(nn.Module):
                           S_prev=torch.zeros(batch, H, hd, hd, device=device),
                           S_intra=torch.zeros(batch, H, hd, hd, device=device), pos=0)
 
-    @staticmethod
-    def _capture_conv(xp, state):
-        n = min(3, xp.shape[1])
-        state.conv.zero_()
-        state.conv[:, 3 - n:].copy_(xp[:, xp.shape[1] - n:])
-        state.S_intra.zero_()
-        state.pos = 0
+    def _prefill_state(self, xp):
+        """The state a prefill over chunk-aligned xp fills in: its last three rows kept here, h and
+        S_prev left to the kernels that write them."""
+        B, L, _ = xp.shape
+        if L < 3 or xp.numel() == 0:
+            state = self.new_state(B, xp.device, xp.dtype)
+            state.conv[:, 3 - L:].copy_(xp)
+            return state
+        H, hd = self.num_heads, self.head_dim
+        f32 = dict(device=xp.device, dtype=torch.float32)
+        return BlockState(conv=xp[:, L - 3:].clone(memory_format=torch.contiguous_format),
+                          h=torch.empty(B, self.d_state, **f32), S_prev=torch.empty(B, H, hd, hd, **f32),
+                          S_intra=torch.zeros(B, H, hd, hd, **f32), pos=0)
 
     def prefill(self, x):
         """Forward over x [B,L,dm] that also returns the BlockState after its last token.
@@ -432,9 +527,11 @@ class HdcMamba9v3Block(nn.Module):
         _ops._on_gpu(x)
         B, L_in, _ = x.shape
         pad = (self.chunk_size - (L_in % self.chunk_size)) % self.chunk_size
-        xp = F.pad(x, (0, 0, pad, 0)).contiguous() if pad else x.contiguous()
-        state = self.new_state(B, x.device, x.dtype)
-        self._capture_conv(xp, state)
+        if pad and not torch.is_grad_enabled() and self._native_ok(x):
+            xp = _ops.native().pad_rows(x, pad, _ops._stream(x))
+        else:
+            xp = F.pad(x, (0, 0, pad, 0)).contiguous() if pad else x.contiguous()
+        state = self._prefill_state(xp.detach())
         y = self._inner_forward(xp, state)
         return y[:, pad:, :], state
 
@@ -444,6 +541,16 @@ class HdcMamba9v3Block(nn.Module):
         state.pos is left to the caller (graph replay)."""
         _ops._on_gpu(x)
         dm, ds, H, C = self.d_model, self.d_state, self.num_heads, self.chunk_size
+        if not torch.is_grad_enabled() and self._native_ok(x):
+            w = self.in_proj.weight
+            front = (self.fused_step_front and x.dtype == torch.bfloat16 and w.shape[0] >= 2048
+                     and 1 <= x.shape[0] <= _ops.SKINNY_MAX_ROWS and dm % 32 == 0 and dm <= 2048)
+            y = _ops.native().block_step(
+                x, self._params(), self.norm.eps, (ds, H, C), state.conv, state.h, state.S_prev, state.S_intra, state.pos,
+                pos_dev, front, self._fused_out(x), _ops.step_workspace(x.device) if front else None, _ops._stream(x))
+            if pos_dev is None:
+                state.pos = (state.pos + 1) % C
+            return y
         B = x.shape[0]
         dtype = x.dtype
         w_in, b_in = self.in_proj.weight.to(dtype), self.in_proj.bias.to(dtype)
@@ -473,15 +580,34 @@ class HdcMamba9v3Block(nn.Module):
             state.pos = (state.pos + 1) % C
         return y
 
+    def _refresh_gamma(self):
+        """gamma_buf from decay_log, as the reference does at every training forward (model.py:390)."""
+        d, g = self.decay_log, self.gamma_buf
+        with torch.no_grad():
+            if (d.dtype == g.dtype and d.dtype in _ops._DTYPES and d.is_cuda and g.device == d.device and d.is_contiguous()
+                    and g.is_contiguous() and not torch.is_autocast_enabled("cuda")):
+                _ops.native().refresh_gamma(d, g, _ops._stream(g))
+            else:
+                g.copy_(torch.exp(-F.softplus(d)))
+
     def forward(self, x):
         _ops._on_gpu(x)
         B, L_in, _ = x.shape
         pad = (self.chunk_size - (L_in % self.chunk_size)) % self.chunk_size
+        if self.training:
+            self._refresh_gamma()
+        if self._native_ok(x):
+            if not torch.is_grad_enabled():
+                return self._native_padded(x, pad), None
+            if self.training:
+                params = self._grad_params()
+                if x.requires_grad or any(p.requires_grad for p in params):
+                    return BlockTrainFunction.apply(self, x, pad, *params), None
+                with torch.no_grad():
+                    return self._native_padded(x, pad), None
         if pad > 0:
             x = F.pad(x, (0, 0, pad, 0))
         if self.training:
-            with torch.no_grad():
-                self.gamma_buf.copy_(torch.exp(-F.softplus(self.decay_log)))
             # the reference checkpoints the block body in training (model.py:391-392): only
             # x is kept for backward and the body runs again when the gradient is needed
             y = checkpoint(self._inner_forward, x.contiguous(), use_reentrant=False)
@@ -556,7 +682,7 @@ class HdcMamba9v3Model(nn.Module):
             for layer in self.layers:
                 if pad:
                     r[:, :pad].zero_()
-                st = layer.new_state(B, x.device, x.dtype)
+                st = layer._prefill_state(r)
                 layer._residual_step_(r, st)
                 states.append(st)
         y = _ops.layer_norm(r[:, pad:].contiguous(), self.norm_final.weight, self.norm_final.bias,

@@ -287,6 +287,31 @@ int hdcm_gnorm_gate_bwd(const void* y, int64_t y_row_stride, const void* gate, i
                         int64_t rows, int64_t dm, int64_t H, int dtype, void* stream);
 
 /*
+ * dst [B, pad + L, D] contiguous: pad zero rows, then src's L rows, per batch row (the left padding
+ * to whole chunks, hdcmamba/model.py:388-389).  Rows 16-byte aligned.
+ */
+int hdcm_pad_rows_fwd(const void* src, int64_t src_batch_stride, int64_t src_row_stride, void* dst, int64_t B, int64_t L,
+                      int64_t pad, int64_t D, int dtype, void* stream);
+
+/*
+ * gamma[h] = exp(-softplus(decay_log[h])), rounded to the dtype after the softplus and after the
+ * exponential (hdcmamba/model.py:327,390).
+ */
+int hdcm_gamma_fwd(const void* decay_log, void* gamma, int64_t H, int dtype, void* stream);
+
+/*
+ * Work issued to `stream` from now on runs after what `after` holds now (an event recorded and
+ * waited for; both streams on `device`).  Allowed while the streams are being captured.
+ */
+int hdcm_stream_after(void* stream, void* after, int device);
+
+/*
+ * Whether hdcm_gemm_fwd is the faster choice for x [M, K] W [N, K]^T + bias against the library's
+ * default solution (1 or 0); the rule and its measurements are in csrc/gemm.hip.
+ */
+int hdcm_gemm_preferred(int64_t M, int64_t N, int64_t K, int dtype);
+
+/*
  * Gradient of hdcm_slot_state_fwd + hdcm_slot_gate_fwd (gamma constant) in two passes: writes the
  * q, k, v and gate column blocks of dprojs (4 dm columns from q_col on, activation dtype) and
  * d gn_w, d gn_b (fp32 [dm], summed in a fixed order) from projs, dout [B*L, dm] and ws_fwd, the

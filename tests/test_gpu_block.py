@@ -4,9 +4,13 @@ import torch
 
 import oracle
 from cfgs import (WORKLOADS, assert_close, assert_close_normwise, block_input, lm_input, make_block, make_lm, max_rel,
-                  oracle_cfg)
+                  oracle_cfg, reinit_block_)
 
 pytestmark = pytest.mark.gpu
+
+
+def _say(*a):
+    print(*a, flush=True)
 
 
 def _sd(m):
@@ -298,3 +302,117 @@ def test_lm_logits_against_oracle(dev, name):
     assert_close_normwise(seen["h"], ref_h, torch.bfloat16, f"{name} head input, every position")
     assert_close_normwise(got, ref, torch.bfloat16, f"{name} logits")
 
+
+
+# ----------------------------------------------------------------- native host path
+def _composition(blk):
+    """blk with the native host path off: the Python composition of the same kernels."""
+    blk._native_ok = lambda x: False
+    return blk
+
+
+@pytest.mark.parametrize("dtype,dm,ds,H,C,B,L", [
+    (torch.bfloat16, 256, 64, 4, 64, 2, 192),   # row statistics from the producers, no padding
+    (torch.bfloat16, 256, 64, 4, 64, 3, 100),   # padded
+    (torch.bfloat16, 64, 8, 2, 8, 1, 13),       # at most 16 rows: statistics inside the GEMM
+    (torch.bfloat16, 100 * 8, 32, 10, 64, 1, 65),  # d_model 800: in_proj on the library GEMM
+    (torch.float32, 256, 64, 8, 64, 2, 100), (torch.float32, 48, 12, 1, 20, 1, 20)])
+def test_native_forward_is_the_composition(dev, dtype, dm, ds, H, C, B, L):
+    """The native host path issues the composition's kernels on the same operands: forward,
+    prefill (output and state) and a decode step are bit-identical; so for every placement of the
+    scan."""
+    from hdcmamba_amd import HdcMamba9v3Block
+
+    _say("native forward", dtype, dm, ds, H, C, B, L)
+    torch.manual_seed(0)
+    blk = reinit_block_(HdcMamba9v3Block(dm, ds, H, C), seed=3, decays_uniform=True).to(dtype).to(dev).eval()
+    g = torch.Generator(device=dev).manual_seed(L)
+    x = torch.randn(B, L, dm, generator=g, device=dev).to(dtype)
+    tok = torch.randn(B, dm, generator=g, device=dev).to(dtype)
+
+    def all_of():
+        with torch.no_grad():
+            y, st = blk.prefill(x)
+            step = blk.step(tok, st)
+            strided = blk(torch.cat([x, x], -1)[..., :dm])[0]
+            return [blk(x)[0], strided, y, step, st.conv, st.h, st.S_prev, st.S_intra]
+
+    got = [all_of()]
+    for mode in ("none", "state", "gate", "after_state"):
+        blk.ssm_overlap = mode
+        got.append(all_of())
+    blk.ssm_overlap = "auto"
+    want = (_composition(blk), all_of())[1]
+    torch.cuda.synchronize()
+    for a in got:
+        for x1, x2 in zip(a, want):
+            assert torch.equal(x1, x2)
+
+
+@pytest.mark.parametrize("dtype,L,mixer", [(torch.bfloat16, 100, True), (torch.float32, 128, True),
+                                           (torch.float32, 100, False)])
+def test_native_training_is_the_composition(dev, dtype, L, mixer):
+    """BlockTrainFunction against autograd through the checkpointed composition: the output, the
+    input's and every parameter's gradient (fp32 sums in another order; bf16 products of the same
+    rounded operands), a frozen parameter, a non-contiguous upstream gradient, and a backward that
+    is differentiated again."""
+    from hdcmamba_amd import HdcMamba9v3Block
+
+    _say("native training", dtype, L, mixer)
+    torch.manual_seed(0)
+    blk = reinit_block_(HdcMamba9v3Block(256, 64, 4, 64, differentiable_mixer=mixer), seed=3, decays_uniform=True)
+    blk = blk.to(dtype).to(dev).train()
+    blk.conv1d.bias.requires_grad_(False)
+    g = torch.Generator(device=dev).manual_seed(L)
+    x = torch.randn(2, L, 256, generator=g, device=dev).to(dtype).requires_grad_()
+    dy = torch.randn(2, 256, L, generator=g, device=dev).to(dtype).transpose(1, 2)
+
+    def grads():
+        blk.zero_grad(set_to_none=True)
+        x.grad = None
+        y, _ = blk(x)
+        y.backward(dy)
+        out = {k: p.grad for k, p in blk.named_parameters()}
+        return {"y": y.detach(), "x": x.grad, "gamma": blk.gamma_buf.clone(), **out}
+
+    def second():  # d/dx of sum(gradient of out_proj^2): linear in dy, so in the graph's own dy
+        d = dy.detach().clone().requires_grad_()
+        y, _ = blk(x)
+        (gw,) = torch.autograd.grad(y, [blk.out_proj.weight], d, create_graph=True)
+        return torch.autograd.grad((gw.float() ** 2).sum(), [d])[0]
+
+    a, a2 = grads(), second()
+    _composition(blk)
+    b, b2 = grads(), second()
+    lim = 1e-5 if dtype == torch.float32 else 1.5e-2
+    assert [k for k in a if a[k] is None] == [k for k in b if b[k] is None]
+    for k in a:
+        if a[k] is not None:
+            assert a[k].dtype == b[k].dtype and a[k].shape == b[k].shape, k
+            assert max_rel(a[k], b[k]) <= lim, (k, max_rel(a[k], b[k]))
+    assert max_rel(a2, b2) <= lim
+    with torch.no_grad():  # training mode without a graph
+        assert not blk(x)[0].requires_grad
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_pad_rows_and_gamma(dev, dtype):
+    """The padding kernel against F.pad (a batch-strided view, no rows of padding, a width of one
+    16-byte group) and the decay kernel against the tensor operations: equal."""
+    from hdcmamba_amd import _ops
+
+    n = _ops.native()
+    s = torch.cuda.current_stream(dev).cuda_stream
+    g = torch.Generator(device=dev).manual_seed(1)
+    full = torch.randn(3, 50, 264, generator=g, device=dev).to(dtype)
+    for x, pad in ((full, 14), (full[:, 7:, 8:136], 21), (full, 0), (full[:1, :1, :8].contiguous(), 255), (full[..., 3:], 4)):
+        assert torch.equal(n.pad_rows(x, pad, s), torch.nn.functional.pad(x, (0, 0, pad, 0)))
+    d = (6 * torch.randn(300, generator=g, device=dev)).to(dtype)
+    d[0], d[1] = 25.0, -30.0
+    gamma = torch.empty_like(d)
+    v = gamma._version
+    n.refresh_gamma(d, gamma, s)
+    ref = torch.exp(-torch.nn.functional.softplus(d))
+    # the same fp32 functions rounded in the same places; their last bits may differ
+    torch.testing.assert_close(gamma, ref, rtol=2e-6 if dtype == torch.float32 else 2 ** -7, atol=0)
+    assert gamma._version == v + 1

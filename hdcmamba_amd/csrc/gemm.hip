@@ -442,10 +442,10 @@ int64_t tiles_of(int64_t M, int64_t N) {
 }
 
 // Tile width (256, 128 or 64) with the least estimated time, in hundredths of a microsecond.
-// Measured per K step of 64: a 256-wide tile, one workgroup per CU, 2.0 us; a 128-wide tile 0.6
-// us alone on its CU and 1.2 us for the two that share one; a 64-wide tile 0.45 us alone, 0.195
-// us per tile once several share the CU; plus 3-5 us per round of workgroups for the prologue
-// and the stores.  A grid of fewer than 256 large tiles leaves CUs idle for a whole large tile's
+// Fitted to measurements: per K step of 64 a 256-wide tile, one workgroup per CU, takes 2.0 us; a
+// 128-wide tile 0.58 us alone on its CU and 1.2 us for the two that share one; a 64-wide tile 0.41
+// us alone, 0.23 us per tile once several share the CU; plus 3.5-6.5 us per round of workgroups
+// for the prologue and the stores.  A grid of fewer than 256 large tiles leaves CUs idle for a whole large tile's
 // K loop.  Out_proj with the folded LayerNorm at K = 832, N = 768: 4096 rows 28.4 us with 256,
 // 14.0 with 128, 12.4 with 64; 8192 rows 29.4, 18.9, 21.8; 32768 rows 70.6, 67.8, 91.3.  In_proj
 // at K = 768, N = 3264: 2048 rows 27.6, 17.4, 21.0; 8192 rows 54.9, 58.5, 71.6; 32768 rows 201,
@@ -456,8 +456,8 @@ int tile_choice(int64_t M, int64_t N, int64_t K) {
   const int64_t c256 = per_cu(tiles_of<Tile256>(M, N)), c128 = per_cu(tiles_of<Tile128>(M, N)),
                 c64 = per_cu(tiles_of<Tile64>(M, N));
   const int64_t t256 = c256 * (200 * nk + 500);
-  const int64_t t128 = c128 / 2 * (120 * nk + 400) + c128 % 2 * (60 * nk + 300);
-  const int64_t t64 = std::max<int64_t>(45 * nk, c64 * nk * 39 / 2) + 300;
+  const int64_t t128 = c128 / 2 * (120 * nk + 350) + c128 % 2 * (58 * nk + 650);
+  const int64_t t64 = std::max<int64_t>(41 * nk, c64 * nk * 23) + 430;
   if (t256 <= t128 && t256 <= t64) return 256;
   return t128 <= t64 ? 128 : 64;
 }

@@ -52,6 +52,10 @@ _PROTOS = {
     "hdcm_gamma_fwd": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "hdcm_stream_after": (c_int, [c_void_p, c_void_p, c_int]),
     "hdcm_gemm_preferred": (c_int, [c_int64, c_int64, c_int64, c_int]),
+    "hdcm_gemm_tn_preferred": (c_int, [c_int64, c_int64, c_int64, c_int, c_int]),
+    "hdcm_gemm_tn_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
+    "hdcm_gemm_tn": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_size_t,
+                             c_int64, c_int64, c_int64, c_int, c_void_p]),
     "hdcm_slot_grad_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int]),
     "hdcm_slot_grad": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_size_t,
                                c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_size_t, c_int64,
@@ -911,6 +915,23 @@ def gemm_preferred(x, weight, bias) -> bool:
             and weight.shape[1] == K and x.is_contiguous() and weight.is_contiguous() and bias.is_contiguous()
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and bias.data_ptr() % 8 == 0
             and not torch.cuda.tunable.is_enabled())
+
+
+def gemm_tn(y_grad, x, col_sums=False):
+    """y_grad [M, N]^T x [M, K] -> [N, K] on the weight-gradient GEMM (bf16, fp32 accumulation), and with
+    ``col_sums`` the column sums of y_grad [N]."""
+    _on_gpu(y_grad, x)
+    M, N = y_grad.shape
+    K = x.shape[1]
+    if x.dtype != y_grad.dtype or x.shape[0] != M:
+        raise RuntimeError("gemm_tn: y_grad [M, N] and x [M, K] must match")
+    out = torch.empty(N, K, device=x.device, dtype=x.dtype)
+    cs = torch.empty(N, device=x.device, dtype=x.dtype) if col_sums else None
+    ws = torch.empty(max(lib().hdcm_gemm_tn_workspace_bytes(M, N, K), 16), dtype=torch.uint8, device=x.device)
+    _check("hdcm_gemm_tn", lib().hdcm_gemm_tn(
+        y_grad.data_ptr(), _rows2d(y_grad, "y_grad"), x.data_ptr(), _rows2d(x, "x"), out.data_ptr(), K,
+        cs.data_ptr() if col_sums else None, ws.data_ptr(), ws.numel(), M, N, K, _dtype(x), _stream(x)))
+    return (out, cs) if col_sums else out
 
 
 def rowln_gemm(c, weight, residual, eps=1e-5, out=None):

@@ -426,6 +426,21 @@ std::vector<Tensor> norm_conv_backward(const Tensor& go_, const Tensor& x_, cons
   return {g.first, w.narrow(0, 0, D), w.narrow(0, D, D), w.narrow(0, 2 * D, 4 * D).view(cw.sizes()), w.narrow(0, 6 * D, D)};
 }
 
+// Weight gradient y^T x of row-major y [M, N], x [M, K] and, with sums, y's column sums
+std::pair<Tensor, Tensor> weight_grad(const Tensor& y, const Tensor& x, bool sums, bool library, void* s) {
+  const int64_t M = y.size(0), N = y.size(1), K = x.size(1);
+  const auto aligned = [](const Tensor& t) { return (uintptr_t)t.const_data_ptr() % 16 == 0; };
+  if (library || !hdcm_gemm_tn_preferred(M, N, K, sums, dtype_of(y)) || !aligned(y) || !aligned(x))
+    return {at::mm(y.t(), x), sums ? y.sum(0) : Tensor()};
+  Tensor w = at::empty({N, K}, y.options()), c = sums ? at::empty({N}, y.options()) : Tensor();
+  const size_t n = hdcm_gemm_tn_workspace_bytes(M, N, K);
+  Tensor ws = bytes(n, y);
+  check("hdcm_gemm_tn", hdcm_gemm_tn(y.const_data_ptr(), N, x.const_data_ptr(), K, w.mutable_data_ptr(), K,
+                                     sums ? c.mutable_data_ptr() : nullptr, ws.mutable_data_ptr(), ws.numel(), M, N, K,
+                                     HDCM_BF16, s));
+  return {w, c};
+}
+
 // Recompute and backward of one block in training from x and dy [B, L, dm] (chunk-aligned,
 // contiguous): gradients of x and of the parameters in params_of's order (undefined where there is
 // none), in the parameters' dtypes.  mixer_grad: the differentiable mixer; otherwise the SSM and slot
@@ -456,7 +471,7 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
   if (need[11]) {
     Tensor c = at::empty_like(m.combined);
     row_norm(m.combined, c, st.main);
-    give(10, at::mm(dy2.t(), c.view({M, K})));
+    give(10, weight_grad(dy2, c.view({M, K}), false, library, st.main).first);
   }
   if (!mixer_grad) {
     if (need[0]) out[0] = dy;
@@ -480,8 +495,13 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
     give(6, w.narrow(0, 2 * dm, d.ds));
   }
   const Tensor dproj2 = g.first.view({M, N});
-  if (need[6]) give(5, dproj2.sum(0));
-  if (need[5]) give(4, at::mm(dproj2.t(), m.x_conv.view({M, dm})));
+  if (need[5]) {
+    const auto wg = weight_grad(dproj2, m.x_conv.view({M, dm}), need[6], library, st.main);
+    give(4, wg.first);
+    if (need[6]) give(5, wg.second);
+  } else if (need[6]) {
+    give(5, dproj2.sum(0));
+  }
   if (need[0] || need[1] || need[2] || need[3] || need[4]) {
     Tensor dxc = at::mm(dproj2, p.w_in).view({B, L, dm});
     auto n = norm_conv_bwd(dxc, x, p.nw, p.nb, p.cw, p.eps, st.main);

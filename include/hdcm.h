@@ -306,6 +306,19 @@ int hdcm_gamma_fwd(const void* decay_log, void* gamma, int64_t H, int dtype, voi
 int hdcm_stream_after(void* stream, void* after, int device);
 
 /*
+ * Weight gradient of y = x W^T + b: out [N, K] = y_grad^T x over M rows (y_grad [M, N], x [M, K], bf16,
+ * fp32 accumulation in a fixed order, one rounding) and, with col_sums, the column sums of y_grad
+ * (bf16 [N], the bias gradient).  N, K multiples of 8, rows 16-byte aligned.  ws:
+ * hdcm_gemm_tn_workspace_bytes bytes, 16-byte aligned.  Replaces: autograd of nn.Linear
+ * (hdcmamba/model.py:313,320).
+ */
+int hdcm_gemm_tn_preferred(int64_t M, int64_t N, int64_t K, int col_sums, int dtype); /* against the library's product */
+size_t hdcm_gemm_tn_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int hdcm_gemm_tn(const void* y_grad, int64_t y_row_stride, const void* x, int64_t x_row_stride, void* out,
+                 int64_t out_row_stride, void* col_sums, void* ws, size_t ws_bytes, int64_t M, int64_t N, int64_t K,
+                 int dtype, void* stream);
+
+/*
  * Whether hdcm_gemm_fwd is the faster choice for x [M, K] W [N, K]^T + bias against the library's
  * default solution (1 or 0); the rule and its measurements are in csrc/gemm.hip.
  */

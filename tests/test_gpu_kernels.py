@@ -769,6 +769,28 @@ def test_gemm_tile_widths(dev, M, N, K):
         assert (err <= 2 ** -8 * ref.abs() + 2e-3).all(), f"{what}: max err {err.max().item()}"
 
 
+@pytest.mark.parametrize("M,N,K,sums", [
+    # one row, fewer rows than a step, rows not a multiple of the step in the last range, one and many
+    # ranges, tiles ragged in both outputs (one group over; less than a tile), more tiles than two per CU
+    (1, 8, 8, True), (31, 264, 136, True), (97, 256, 128, False), (1000, 520, 8, True), (2049, 768, 832, False),
+    (5000, 2240, 512, True), (4097, 3264, 768, True), (700, 8576, 2048, True)])
+def test_gemm_tn(dev, M, N, K, sums):
+    """The weight-gradient GEMM and its column sums against fp64 on the same bf16 operands: one bf16
+    rounding and an fp32 sum of M products of size ~1 (2e-6 sqrt(M) of the result's scale sqrt(M))."""
+    _say("gemm_tn", M, N, K, sums)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    big = torch.randn(M, N + K + 16, generator=g, device=dev).to(torch.bfloat16)
+    y, x = big[:, 8:8 + N], big[:, 8 + N:8 + N + K]  # strided rows
+    out = _ops.gemm_tn(y, x, sums)
+    ref = y.double().t() @ x.double()
+    got = out[0] if sums else out
+    err = (got.double() - ref).abs() - 2 ** -8 * ref.abs()
+    assert err.max() <= 2e-6 * M + 1e-6, err.max().item()
+    if sums:
+        cs = y.double().sum(0)
+        assert ((out[1].double() - cs).abs() - 2 ** -8 * cs.abs()).max() <= 2e-6 * M + 1e-6
+
+
 def test_fused_out_proj_matches_unfused(dev):
     """A bf16 model forward with the LayerNorm folded into out_proj against the same model
     with the row LayerNorm kernel and addmm."""

@@ -1,6 +1,6 @@
 // Backward of the fused LayerNorm + causal depthwise conv (width 4) for gfx950.
 //
-// Forward (norm_conv.hip; hdcmamba/model.py:22-72): xh[t] = (x[t] - mu_t) * r_t,
+// Forward (norm_conv_kernels.h; hdcmamba/model.py:22-72): xh[t] = (x[t] - mu_t) * r_t,
 // u[t] = xh[t] * g + b for t >= 0 and u[t] = b for t < 0 (the LayerNorm of a zero row),
 // out[t] = sum_k w_k u[t-3+k] + cb.  With go = dL/dout this computes the exact gradients
 // of that forward (hdcmamba/model.py:74-166 is the reference's backward, which drops the

@@ -35,6 +35,15 @@ def test_norm_conv(dev, dtype, D, L):
     assert_close(out, ref, dtype, "norm_conv")
 
 
+@pytest.mark.parametrize("dtype,D,L", [(torch.bfloat16, 768, 4096), (torch.bfloat16, 768, 4105), (torch.bfloat16, 1024, 4112),
+                                       (torch.float32, 520, 4101), (torch.float32, 2048, 4099)])
+def test_norm_conv_long_runs(dev, dtype, D, L):
+    """8192 rows (the last size with 4-row runs) and just above (16-row runs, the last one whole or
+    partial), with and without idle lanes."""
+    _say("norm_conv long runs", dtype, D, L)
+    test_norm_conv(dev, dtype, D, L)
+
+
 @pytest.mark.parametrize("D,L", [(2560, 50), (4096, 37), (6144, 19)])
 def test_norm_conv_wide_rows_bf16(dev, D, L):
     """bf16 rows wider than 32 columns per lane take the one-row-at-a-time path (up to the 6144

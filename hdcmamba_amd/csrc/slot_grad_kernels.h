@@ -164,7 +164,7 @@ struct GradArgs {
   T *o1, *o2, *dy;         // d gate or d v; d q or d k; dy (FWD)
   int64_t o_rs, dy_rs;
   const T *gamma, *gn_w, *gn_b;
-  const float* Ain;        // segment-start states
+  const float *Ain, *Win;  // segment-start states A and (null: zero) W
   float* part;             // FWD: [B * nseg][2][H * HD] partial sums of d gn_w, d gn_b
   float gn_eps;
   int L, C, cshift, conf, seg_rows, nseg;
@@ -204,15 +204,18 @@ __global__ __launch_bounds__(kThreads, HD > 64 ? 1 : 2) void slot_grad_kernel(co
 
   f32x4_t stA[OWN][NVT];
   f32x4_t stW[HAS_W ? OWN : 1][HAS_W ? NVT : 1];
-  const float* ain = A.Ain + (((int64_t)bb * H + h) * A.nseg + seg) * HD * HD;
+  const int64_t st0 = (((int64_t)bb * H + h) * A.nseg + seg) * HD * HD;
 #pragma unroll
   for (int ov = 0; ov < OWN; ++ov) {
     const int vt = w + kWaves * ov;
 #pragma unroll
     for (int mt = 0; mt < NVT; ++mt) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) stA[ov][mt][r] = vt < NVT ? ain[(mt * 16 + kg * 4 + r) * HD + vt * 16 + l16] : 0.f;
-      if constexpr (HAS_W) stW[ov][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int r = 0; r < 4; ++r) {
+        const int64_t e = st0 + (mt * 16 + kg * 4 + r) * HD + vt * 16 + l16;
+        stA[ov][mt][r] = vt < NVT ? A.Ain[e] : 0.f;
+        if constexpr (HAS_W) stW[ov][mt][r] = A.Win != nullptr && vt < NVT ? A.Win[e] : 0.f;
+      }
     }
   }
 
@@ -589,7 +592,7 @@ int launch_grad(const hdcm_slot::GradCall& g, const SlotPlan& pl, hipStream_t s)
   A.o1 = dq + 3 * dm, A.o2 = dq, A.o_rs = g.dprs;
   A.dy = (T*)g.dy, A.dy_rs = dm;
   A.gamma = (const T*)g.gamma, A.gn_w = (const T*)g.gn_w, A.gn_b = (const T*)g.gn_b, A.gn_eps = g.gn_eps;
-  A.Ain = (const float*)g.ws_fwd + (size_t)g.B * g.H * pl.nseg * HD * HD;
+  A.Ain = slot_ws_a(g.ws_fwd, g.B, g.H, pl), A.Win = slot_ws_w(g.ws_fwd, g.B, g.H, pl);
   A.part = g.part;
   A.L = (int)g.L, A.C = (int)g.C, A.cshift = pl.cshift, A.conf = pl.conf, A.seg_rows = pl.seg_rows, A.nseg = pl.nseg;
   if (pl.has_w) HDCM_LAUNCH((slot_grad_kernel<T, HD, TC, true, true>), grid, dim3(kThreads), 0, s, A);
@@ -604,7 +607,6 @@ int launch_grad(const hdcm_slot::GradCall& g, const SlotPlan& pl, hipStream_t s)
   const T* q_end = q + (rows - 1) * g.prs;
   T* dq_end = dq + (rows - 1) * g.dprs;
   float* U = (float*)g.ws_rev;
-  float* Ain = U + (size_t)g.B * g.H * pl.nseg * HD * HD;
   if (pl.nseg > 1) {
     HDCM_LAUNCH((slot_state_kernel<T, HD, TC, true, true>), dim3((unsigned)g.H, pl.nseg - 1, (unsigned)g.B),
                 dim3(kThreads), 0, s, q_end, -g.prs, 0, 0, (int)g.L, (const T*)g.gamma, pl.seg_rows, pl.nseg, U,
@@ -612,14 +614,12 @@ int launch_grad(const hdcm_slot::GradCall& g, const SlotPlan& pl, hipStream_t s)
     st = hdcm_launch_status();
     if (st) return st;
   }
-  HDCM_LAUNCH((slot_scan_kernel<T>), dim3((HD * HD + kThreads - 1) / kThreads, (unsigned)g.H, (unsigned)g.B),
-              dim3(kThreads), 0, s, U, (const float*)nullptr, Ain, (const T*)g.gamma, HD * HD, pl.nseg, pl.seg_rows);
-  st = hdcm_launch_status();
+  st = launch_scan<T>(nullptr, U, g.gamma, g.B, g.H, pl, s);
   if (st) return st;
   A.a = q_end + dm, A.b = q_end, A.v = dy_end, A.e = q_end + 2 * dm;
   A.prs = -g.prs, A.vrs = -dm;
   A.o1 = dq_end + 2 * dm, A.o2 = dq_end + dm, A.o_rs = -g.dprs;
-  A.Ain = Ain;
+  A.Ain = slot_ws_a(U, g.B, g.H, pl), A.Win = slot_ws_w(U, g.B, g.H, pl);
   if (pl.has_w) HDCM_LAUNCH((slot_grad_kernel<T, HD, TC, true, false>), grid, dim3(kThreads), 0, s, A);
   else HDCM_LAUNCH((slot_grad_kernel<T, HD, TC, false, false>), grid, dim3(kThreads), 0, s, A);
   return hdcm_launch_status();

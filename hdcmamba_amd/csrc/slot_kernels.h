@@ -27,11 +27,12 @@
 // columns up to the next multiple of 32 (written once per workgroup); contractions over
 // tokens and the value columns use the hd/16 16-wide tiles as they are.
 //
-// Parallelism: the sequence is cut into segments of whole tiles that start on chunk
-// boundaries.  slot_state_kernel computes each segment's contribution U_s to A (from k
-// and v only), slot_scan_kernel turns them into the state at every segment start, and
-// slot_gate_kernel walks each (batch, head, segment) with its own start state.  That
-// gives B*H*nseg workgroups instead of the reference's B*H serial programs.
+// Parallelism: the sequence is cut into segments of whole tiles that start on chunk boundaries or,
+// for chunks of several whole tiles, divide a chunk evenly.  slot_state_kernel computes each
+// segment's contribution U_s to A and W (from k and v only), slot_scan_kernel turns them into the
+// states at every segment start (W too where segments divide chunks), and slot_gate_kernel walks
+// each (batch, head, segment) with its own start states.  That gives B*H*nseg workgroups instead
+// of the reference's B*H serial programs.
 //
 // MFMA mapping (v_mfma_f32_16x16x32_bf16; fp32 uses 8x v_mfma_f32_16x16x4f32).  A C/D
 // tile puts column n = lane%16 and rows 4*(lane/16)+r in a lane.  Scores are computed
@@ -64,7 +65,13 @@ constexpr int kWaves = kThreads / kWave;
 // 1.3 rounds of the gate pass at 3 workgroups per CU) and to 4-13 or 22.
 constexpr int kTargetWorkgroups = 512;
 constexpr int kGateWavesPerEU = 3;  // register budget: 3 waves per SIMD (3 workgroups per CU)
-constexpr int kMinSegTiles = 4;
+// Fewest tiles per segment: 4, or 2 where 4 leave less than a workgroup per CU and a segment's
+// serial tiles are the kernel's time (state + scan + gate, bf16: B=2 L=1024 12 heads of 64 21.6
+// us with 4, 16.0 with 2, 17.8 with 1; B=4 L=2048 8 heads of 96, 256 workgroups of 4, 39.4 and
+// 45.7 with 2; fp32, B=8 L=256 8 heads of 64 31.0 and 21.9).  Segments that divide a chunk count
+// alike (B=2 L=1024, 8 heads of 64, chunk 256: bf16 23.7 in whole chunks, 16.6 in halves; fp32
+// 53.1, 23.8 in quarters).
+constexpr int kMinSegTiles = 4, kFewSegTiles = 2, kCus = 256;
 
 template <typename T>
 struct TileOf {
@@ -385,7 +392,7 @@ template <typename T, int HD, int TC, bool HAS_W, bool PAIRS, bool PHI, bool EPI
 __global__ __launch_bounds__(kThreads, HD > 64 ? 1 : (HAS_W ? 2 : kGateWavesPerEU)) void slot_gate_kernel(
     const T* __restrict__ projs, int64_t prs, int q_col, int k_off, int v_off, int g_off, int L, int C, int cshift,
     const T* __restrict__ gamma, const T* __restrict__ gn_w, const T* __restrict__ gn_b,
-    float gn_eps, const float* __restrict__ Ain, int seg_rows, int nseg, T* __restrict__ out,
+    float gn_eps, const float* __restrict__ Ain, const float* __restrict__ Win, int seg_rows, int nseg, T* __restrict__ out,
     int64_t ors, int out_col, float* __restrict__ S_final, float* __restrict__ row_stats, int64_t stats_ps,
     const T* __restrict__ zb = nullptr, int64_t zrs = 0) {
   using LD = Lds<T, HD, TC>;
@@ -430,16 +437,19 @@ __global__ __launch_bounds__(kThreads, HD > 64 ? 1 : (HAS_W ? 2 : kGateWavesPerE
   // dk = 16*mt + 4*kg + r, dv = 16*vt + l16.
   f32x4_t stA[OWN][NVT];
   f32x4_t stW[HAS_W ? OWN : 1][HAS_W ? NVT : 1];
-  const float* ain = Ain + (((int64_t)b * H + h) * nseg + seg) * HD * HD;
+  const int64_t st0 = (((int64_t)b * H + h) * nseg + seg) * HD * HD;
 #pragma unroll
   for (int ov = 0; ov < OWN; ++ov) {
     const int vt = w + kWaves * ov;
 #pragma unroll
     for (int mt = 0; mt < NVT; ++mt) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        stA[ov][mt][r] = vt < NVT ? ain[(mt * 16 + kg * 4 + r) * HD + vt * 16 + l16] : 0.f;
-      if constexpr (HAS_W) stW[ov][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int r = 0; r < 4; ++r) {
+        const int64_t e = st0 + (mt * 16 + kg * 4 + r) * HD + vt * 16 + l16;
+        stA[ov][mt][r] = vt < NVT ? Ain[e] : 0.f;
+        // W at the segment's start: zero (Win null) where segments are whole chunks
+        if constexpr (HAS_W) stW[ov][mt][r] = Win != nullptr && vt < NVT ? Win[e] : 0.f;
+      }
     }
   }
 
@@ -863,13 +873,14 @@ __global__ __launch_bounds__(kThreads, HD > 64 ? 2 : 4) void slot_state_kernel(c
   }
 }
 
-// Per (element, head, batch): Ain[s] = state at the start of segment s.
+// Per (element, head, batch): Ain[s] = state A at the start of segment s and, where spc > 1 segments
+// divide a chunk, Win[s] = W there (spc == 1: every segment starts a chunk, W = 0).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void slot_scan_kernel(const float* __restrict__ U,
                                                              const float* __restrict__ S0,
-                                                             float* __restrict__ Ain,
+                                                             float* __restrict__ Ain, float* __restrict__ Win,
                                                              const T* __restrict__ gamma, int HD2,
-                                                             int nseg, int seg_len) {
+                                                             int nseg, int seg_len, int spc) {
   const int e = blockIdx.x * kThreads + threadIdx.x;
   const int h = blockIdx.y, b = blockIdx.z, H = gridDim.y;
   if (e >= HD2) return;
@@ -877,6 +888,7 @@ __global__ __launch_bounds__(kThreads) void slot_scan_kernel(const float* __rest
   const T graw = gamma[h];
   const float* u = U + bh * nseg * HD2 + e;
   float* o = Ain + bh * nseg * HD2 + e;
+  float* ow = Win + bh * nseg * HD2 + e;
   // Segments in batches of kU whose loads are all in flight before the recurrence uses them.
   // The first batch is straight-line code issued before S0 is loaded and gamma used, so no
   // wait precedes its loads; U[s] is needed only for s + 1 < nseg.
@@ -884,24 +896,34 @@ __global__ __launch_bounds__(kThreads) void slot_scan_kernel(const float* __rest
   float uu[kU];
 #pragma unroll
   for (int k = 0; k < kU; ++k) uu[k] = (k + 1 < nseg) ? u[(int64_t)k * HD2] : 0.f;
-  float a = S0 ? S0[bh * HD2 + e] : 0.f;
-  const float gs = fexp2((float)seg_len * log2f(to_f<T>(graw)));
+  float a = S0 ? S0[bh * HD2 + e] : 0.f, w = 0.f;
+  const float lg2 = log2f(to_f<T>(graw));
+  const float gs = fexp2((float)seg_len * lg2), gC = fexp2((float)seg_len * (float)spc * lg2);
+  int left = spc;  // segments to the chunk's end (spc > 1)
+  auto step = [&](int s, float v) {
+    o[(int64_t)s * HD2] = a;
+    if (spc == 1) {
+      a = a * gs + v;
+    } else {
+      ow[(int64_t)s * HD2] = w;
+      w = w * gs + v;
+      if (--left == 0) {
+        a = a * gC + w;
+        w = 0.f;
+        left = spc;
+      }
+    }
+  };
 #pragma unroll
   for (int k = 0; k < kU; ++k) {
-    if (k < nseg) {
-      o[(int64_t)k * HD2] = a;
-      a = a * gs + uu[k];
-    }
+    if (k < nseg) step(k, uu[k]);
   }
   for (int s = kU; s < nseg; s += kU) {
 #pragma unroll
     for (int k = 0; k < kU; ++k) uu[k] = (s + k + 1 < nseg) ? u[(int64_t)(s + k) * HD2] : 0.f;
 #pragma unroll
     for (int k = 0; k < kU; ++k) {
-      if (s + k < nseg) {
-        o[(int64_t)(s + k) * HD2] = a;
-        a = a * gs + uu[k];
-      }
+      if (s + k < nseg) step(s + k, uu[k]);
     }
   }
 }
@@ -914,6 +936,7 @@ struct SlotPlan {
   int HD, TC, seg_rows, nseg, cshift;
   bool has_w;
   bool conf;  // chunk-confined tiles: C neither divides TC nor is a multiple of it
+  int spc;    // segments per chunk (1: segments are whole chunks)
 };
 }  // namespace hdcm_slot
 
@@ -945,18 +968,27 @@ int slot_plan(int64_t B, int64_t L, int64_t dm, int64_t H, int64_t C, int dtype,
     const int64_t bh = B * H > 0 ? B * H : 1;
     const int64_t want = (kTargetWorkgroups + bh - 1) / bh;
     st = (tiles + want - 1) / want;
-    if (st < kMinSegTiles) st = kMinSegTiles;
+    const int64_t least = bh * ((tiles + kMinSegTiles - 1) / kMinSegTiles) < kCus ? kFewSegTiles : kMinSegTiles;
+    if (st < least) st = least;
   }
   if (st < 1) st = 1;
-  // segments start on chunk boundaries: whole TC-row tiles (C dividing TC), else whole chunks
+  // segments: whole TC-row tiles (C dividing TC), else whole chunks, or the largest part of a
+  // chunk of several whole tiles that divides it into segments of at most st tiles
   int64_t seg_rows;
+  pl->spc = 1;
   if (cshift < 31) {
     seg_rows = st * TC;
   } else {
     const int64_t tpc = (C + TC - 1) / TC;  // tiles per chunk
     seg_rows = (st + tpc - 1) / tpc * C;
+    if (C % TC == 0 && st < tpc) {
+      int64_t d = st;
+      while (tpc % d) --d;
+      pl->spc = (int)(tpc / d);
+      seg_rows = d * TC;
+    }
   }
-  if (L > 0 && seg_rows > L) seg_rows = cshift < 31 ? tiles * TC : L;
+  if (L > 0 && seg_rows > L) seg_rows = cshift < 31 ? tiles * TC : L;  // (a part of a chunk is below L)
   if (seg_rows < 1) seg_rows = 1;
   pl->HD = (int)HD;
   pl->TC = TC;
@@ -970,8 +1002,24 @@ int slot_plan(int64_t B, int64_t L, int64_t dm, int64_t H, int64_t C, int dtype,
   return HDCM_OK;
 }
 
+// U, A at the segment starts and, where segments divide chunks, W there
 size_t slot_ws_bytes(int64_t B, int64_t H, const SlotPlan& pl) {
-  return (size_t)2 * B * H * pl.nseg * pl.HD * pl.HD * sizeof(float);
+  return (size_t)(pl.spc > 1 ? 3 : 2) * B * H * pl.nseg * pl.HD * pl.HD * sizeof(float);
+}
+const float* slot_ws_a(const void* ws, int64_t B, int64_t H, const SlotPlan& pl) {
+  return (const float*)ws + (size_t)B * H * pl.nseg * pl.HD * pl.HD;
+}
+const float* slot_ws_w(const void* ws, int64_t B, int64_t H, const SlotPlan& pl) {
+  return pl.spc > 1 ? slot_ws_a(ws, B, H, pl) + (size_t)B * H * pl.nseg * pl.HD * pl.HD : nullptr;
+}
+template <typename T>
+int launch_scan(const float* S0, void* ws, const void* gamma, int64_t B, int64_t H, const SlotPlan& pl, hipStream_t s) {
+  const int hd2 = pl.HD * pl.HD;
+  float* A = const_cast<float*>(slot_ws_a(ws, B, H, pl));
+  HDCM_LAUNCH((slot_scan_kernel<T>), dim3((hd2 + kThreads - 1) / kThreads, (unsigned)H, (unsigned)B), dim3(kThreads), 0, s,
+              (const float*)ws, S0, A, pl.spc > 1 ? const_cast<float*>(slot_ws_w(ws, B, H, pl)) : A, (const T*)gamma, hd2,
+              pl.nseg, pl.seg_rows, pl.spc);
+  return hdcm_launch_status();
 }
 
 // k at column k_col of each row, v v_off columns after k; PHI as in the kernels.
@@ -981,7 +1029,6 @@ int launch_state(const void* base, int64_t prs, int64_t k_col, int64_t v_off, co
                  hipStream_t s) {
   constexpr int TC = TileOf<T>::value;
   float* U = (float*)ws;
-  float* Ain = U + (size_t)B * H * pl.nseg * HD * HD;
   if (pl.nseg > 1) {
     HDCM_LAUNCH((slot_state_kernel<T, HD, TC, PHI>), dim3((unsigned)H, pl.nseg - 1, (unsigned)B),
                        dim3(kThreads), 0, s, (const T*)base, prs, (int)k_col, (int)v_off, (int)L,
@@ -989,10 +1036,7 @@ int launch_state(const void* base, int64_t prs, int64_t k_col, int64_t v_off, co
     const int st = hdcm_launch_status();
     if (st) return st;
   }
-  HDCM_LAUNCH((slot_scan_kernel<T>), dim3((HD * HD + kThreads - 1) / kThreads, (unsigned)H, (unsigned)B),
-                     dim3(kThreads), 0, s, U, S0, Ain, (const T*)gamma, HD * HD, pl.nseg,
-                     pl.seg_rows);
-  return hdcm_launch_status();
+  return launch_scan<T>(S0, ws, gamma, B, H, pl, s);
 }
 
 // q at column q_col of each row; k, v and the gate k_off, v_off, g_off columns after q.
@@ -1003,7 +1047,7 @@ int launch_gate(const void* base, int64_t prs, int64_t q_col, int64_t k_off, int
                 int64_t L, int64_t H, int64_t C, const SlotPlan& pl, hipStream_t s, const void* zb = nullptr,
                 int64_t zrs = 0) {
   constexpr int TC = TileOf<T>::value;
-  const float* Ain = (const float*)ws + (size_t)B * H * pl.nseg * HD * HD;
+  const float *Ain = slot_ws_a(ws, B, H, pl), *Win = slot_ws_w(ws, B, H, pl);
   // heads vary fastest so the workgroups that run together read the same rows of projs
   dim3 grid((unsigned)H, pl.nseg, (unsigned)B);
   // 16-byte output runs need 16-byte aligned rows and columns (bf16 only; fp32 always has them)
@@ -1013,7 +1057,7 @@ int launch_gate(const void* base, int64_t prs, int64_t q_col, int64_t k_off, int
 #define HDCM_GATE_LAUNCH(W, P, CF)                                                                          \
   HDCM_LAUNCH((slot_gate_kernel<T, HD, TC, W, P, PHI, EPI, CHAIN, CF>), grid, dim3(kThreads), 0, s,    \
                      (const T*)base, prs, (int)q_col, (int)k_off, (int)v_off, (int)g_off, (int)L, (int)C,  \
-                     pl.cshift, (const T*)gamma, (const T*)gn_w, (const T*)gn_b, gn_eps, Ain, pl.seg_rows,   \
+                     pl.cshift, (const T*)gamma, (const T*)gn_w, (const T*)gn_b, gn_eps, Ain, Win, pl.seg_rows,   \
                      pl.nseg, (T*)out, ors, (int)out_col, S_final, row_stats, stats_ps, (const T*)zb, zrs)
   // chunk-confined tiles (rare chunk sizes) run with the 8-byte output runs only
   if (pl.conf) {

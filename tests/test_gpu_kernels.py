@@ -385,6 +385,32 @@ def test_slot_segments_option(dev, C, L):
     assert_close(outs[0][..., ds:], ref, torch.float32, "slot+gate")
 
 
+@pytest.mark.parametrize("dtype,B,L,dm,H,C,st", [
+    (torch.bfloat16, 2, 512, 256, 4, 256, 1), (torch.bfloat16, 1, 768, 192, 2, 256, 3),  # 3 of 4 tiles -> 2
+    (torch.bfloat16, 1, 576, 96, 2, 192, 2), (torch.bfloat16, 1, 2304, 256, 2, 128, 1),  # 2 of 3 -> 1; 36 segments
+    (torch.bfloat16, 3, 1024, 32, 2, 1024, 0),                                           # one chunk, automatic
+    (torch.float32, 2, 256, 256, 4, 128, 2), (torch.float32, 1, 64, 128, 1, 64, 1),
+])
+def test_slot_segments_within_chunks(dev, dtype, B, L, dm, H, C, st):
+    """Segments that divide a chunk (both states given at each start) against the oracle, and, from a
+    given state, the state after the last row against segments of whole chunks (fp32 sums in another
+    order: both products of the state stay below 2^-14 of its largest value)."""
+    ds = 64
+    _say("slot segments within chunks", dtype, B, L, dm, H, C, st)
+    projs, gamma, gn_w, gn_b = slot_inputs(B, L, dm, ds, H, dtype, seed=L + dm + C)
+    y, S = oracle.slot_chunked(projs, gamma, dm, ds, H, C, dtype)
+    ref = oracle.gnorm_gate(y, projs[..., 3 * ds + 3 * dm:], gn_w, gn_b, H).to(dtype)
+    S0 = torch.randn(B, H, dm // H, dm // H, generator=torch.Generator().manual_seed(st)).to(dev)
+    with _ops.option("slot_seg_tiles", st):
+        out, _ = _run_slot(dev, projs, gamma, gn_w, gn_b, dm, ds, H, C)
+        out0, sf0 = _run_slot(dev, projs, gamma, gn_w, gn_b, dm, ds, H, C, S0=S0)
+    with _ops.option("slot_seg_tiles", 4096):
+        whole, sfw = _run_slot(dev, projs, gamma, gn_w, gn_b, dm, ds, H, C, S0=S0)
+    assert_close(out[..., ds:], ref, dtype, "slot+gate")
+    assert_close(out0, whole.cpu(), dtype, "slot+gate from S0")
+    assert ((sf0 - sfw).abs().max() / sfw.abs().max()).item() <= 2 ** -14
+
+
 @pytest.mark.parametrize("dm,H", [(200, 5), (576, 4)])  # hd 40 (not a multiple of 16), hd 144
 def test_slot_unsupported_head_dim(dev, dm, H):
     projs, gamma, gn_w, gn_b = slot_inputs(1, 64, dm, 64, H, torch.bfloat16)

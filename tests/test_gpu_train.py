@@ -322,3 +322,13 @@ def test_slot_gradient_passes(dev, dtype, B, L, H, hd, ds, C, seg):
         err = max_rel(x, ref)
         _say(f"  {name}: {err:.2e}")
         assert err <= lim, (name, err)
+
+
+@pytest.mark.parametrize("dtype,B,L,H,hd,ds,C,seg", [
+    (torch.bfloat16, 1, 512, 2, 64, 8, 256, 1), (torch.bfloat16, 1, 384, 1, 96, 8, 192, 2),
+    (torch.bfloat16, 2, 512, 1, 32, 8, 512, 0), (torch.float32, 1, 256, 2, 64, 4, 128, 2),
+    (torch.float32, 1, 192, 1, 48, 4, 64, 1),
+])
+def test_slot_gradient_segments_within_chunks(dev, dtype, B, L, H, hd, ds, C, seg):
+    """The same gradients with segments that divide a chunk, in both directions."""
+    test_slot_gradient_passes(dev, dtype, B, L, H, hd, ds, C, seg)

@@ -60,19 +60,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
-// Segments are sized for about two workgroups per CU (512 on 256 CUs).  At B=1, L=32768,
-// 16 heads the measured forward prefers 16 tiles per segment (512 workgroups) to 8 (1024,
-// 1.3 rounds of the gate pass at 3 workgroups per CU) and to 4-13 or 22.
-constexpr int kTargetWorkgroups = 512;
 constexpr int kGateWavesPerEU = 3;  // register budget: 3 waves per SIMD (3 workgroups per CU)
-// Fewest tiles per segment: 4, or 2 where 4 leave less than a workgroup per CU and a segment's
-// serial tiles are the kernel's time (state + scan + gate, bf16: B=2 L=1024 12 heads of 64 21.6
-// us with 4, 16.0 with 2, 17.8 with 1; B=4 L=2048 8 heads of 96, 256 workgroups of 4, 39.4 and
-// 45.7 with 2; fp32, B=8 L=256 8 heads of 64 31.0 and 21.9).  Segments that divide a chunk count
-// alike (B=2 L=1024, 8 heads of 64, chunk 256: bf16 23.7 in whole chunks, 16.6 in halves; fp32
-// 53.1, 23.8 in quarters).
-constexpr int kMinSegTiles = 4, kFewSegTiles = 2, kCus = 256;
-
 template <typename T>
 struct TileOf {
   static constexpr int value = sizeof(T) == 2 ? 64 : 32;
@@ -946,6 +934,43 @@ using hdcm_slot::SlotPlan;
 // Supported head dims: multiples of 16 up to 128.
 inline bool slot_head_dim_ok(int64_t hd) { return hd >= 16 && hd <= 128 && hd % 16 == 0; }
 
+// Tiles per segment of B*H = bh sequences of `tiles` tiles each, for the state, scan and gate passes
+// together (the gradient passes have the gate's shape).  Only a segment that is the shortest with at
+// most 1, 2, 3 or 4 workgroups per CU can be best: one workgroup more puts a whole segment on top
+// of the busiest CU (bf16, B=8 L=4096, 12 heads of 64: 576 workgroups of 11 tiles 84 us, 768 of 8
+// 73.5, 480 of 13 75.3).  Among those the least cost below, in quarters of a microsecond, fitted to
+// measured times: a tile takes a CU's latency when a workgroup is alone on it and its share of the
+// bandwidth beside others (heads above 64: one gate workgroup per CU), a workgroup its start, and the
+// scan grows with their number.  Measured against 512 workgroups of at least 4 tiles (state + scan +
+// gate): bf16, 12 heads of 64, B=8 L=4096 88 -> 75 us, B=32 L=1024 77 -> 70, B=3 L=8192 70 -> 59; fp32,
+// B=8 L=2048 12 heads 142 -> 128, chunk 256 156 -> 128; small: bf16 B=2 L=1024 12 heads 22.5 -> 16.8,
+// fp32 B=8 L=256 8 heads 32.2 -> 22.4, chunk 256 B=2 L=1024 8 heads 53.1 -> 23.8; unchanged where 512
+// was best (B=1 L=32768 16 heads: 16 tiles; B=4 L=2048 8 heads of 96: 4).  tpc: tiles per chunk, of
+// which a segment holds a whole number or, with `parts`, that it divides evenly.
+int64_t segment_tiles(int64_t bh, int64_t tiles, int64_t tpc, bool parts, int64_t HD) {
+  constexpr int64_t kCus = 256;
+  int64_t best = 0, best_cost = 0;
+  for (int64_t r = (bh + kCus - 1) / kCus, last = r < 2 ? 4 : r + 2; r <= last; ++r) {
+    int64_t n = kCus * r / bh;
+    if (n > tiles) n = tiles;
+    int64_t st = (tiles + n - 1) / n;
+    if (st >= tpc) {
+      st = (st + tpc - 1) / tpc * tpc;
+    } else if (parts) {
+      while (tpc % st) ++st;
+    } else {
+      st = tpc;
+    }
+    n = (tiles + st - 1) / st;
+    const int64_t per_cu = (n * bh + kCus - 1) / kCus;
+    const int64_t gate = (HD > 64 ? 10 : 7) * per_cu, state = 3 * per_cu;
+    int64_t cost = st * (gate > 10 ? gate : 10) + 5 * per_cu + 12 * n * bh / kCus;
+    if (n > 1) cost += st * (state > 4 ? state : 4) + 5 * per_cu;
+    if (best == 0 || cost < best_cost) best = st, best_cost = cost;
+  }
+  return best;
+}
+
 int slot_plan(int64_t B, int64_t L, int64_t dm, int64_t H, int64_t C, int dtype, SlotPlan* pl) {
   if (dtype != HDCM_F32 && dtype != HDCM_BF16) return HDCM_EUNSUPPORTED;
   if (B < 0 || L < 0 || dm <= 0 || H <= 0 || C <= 0 || dm % H) return HDCM_EINVAL;
@@ -964,13 +989,8 @@ int slot_plan(int64_t B, int64_t L, int64_t dm, int64_t H, int64_t C, int dtype,
   if (B > 65535 || H > 65535) return HDCM_EUNSUPPORTED;
   const int64_t tiles = (L + TC - 1) / TC;
   int64_t st = hdcm_option_value(HDCM_OPT_SLOT_SEG_TILES);  // 0: automatic
-  if (st == 0) {
-    const int64_t bh = B * H > 0 ? B * H : 1;
-    const int64_t want = (kTargetWorkgroups + bh - 1) / bh;
-    st = (tiles + want - 1) / want;
-    const int64_t least = bh * ((tiles + kMinSegTiles - 1) / kMinSegTiles) < kCus ? kFewSegTiles : kMinSegTiles;
-    if (st < least) st = least;
-  }
+  const int64_t tpc = cshift < 31 ? 1 : (C + TC - 1) / TC;  // tiles per chunk
+  if (st == 0 && B > 0 && L > 0) st = segment_tiles(B * H, cshift < 31 ? tiles : L / C * tpc, tpc, C % TC == 0, HD);
   if (st < 1) st = 1;
   // segments: whole TC-row tiles (C dividing TC), else whole chunks, or the largest part of a
   // chunk of several whole tiles that divides it into segments of at most st tiles
@@ -979,7 +999,6 @@ int slot_plan(int64_t B, int64_t L, int64_t dm, int64_t H, int64_t C, int dtype,
   if (cshift < 31) {
     seg_rows = st * TC;
   } else {
-    const int64_t tpc = (C + TC - 1) / TC;  // tiles per chunk
     seg_rows = (st + tpc - 1) / tpc * C;
     if (C % TC == 0 && st < tpc) {
       int64_t d = st;

@@ -52,6 +52,9 @@ _PROTOS = {
     "hdcm_gamma_fwd": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "hdcm_stream_after": (c_int, [c_void_p, c_void_p, c_int]),
     "hdcm_gemm_preferred": (c_int, [c_int64, c_int64, c_int64, c_int]),
+    "hdcm_gemm_f32_preferred": (c_int, [c_int64, c_int64, c_int64]),
+    "hdcm_gemm_f32_fwd": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
+                                  c_int64, c_int64, c_int64, c_void_p]),
     "hdcm_gemm_tn_preferred": (c_int, [c_int64, c_int64, c_int64, c_int, c_int]),
     "hdcm_gemm_tn_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
     "hdcm_gemm_tn": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_size_t,
@@ -902,6 +905,37 @@ def gemm(x, weight, bias=None, out=None):
         o2.data_ptr(), o2.stride(0), M, N, K, _dtype(x), _stream(x)))
     timer.end("gemm", ev)
     return out
+
+
+def gemm_f32(x, weight, bias=None, res=None, out=None):
+    """x [M, K] @ weight[N, K]^T (+ bias[N]) (+ res[M, N]) -> [M, N] on the tiled fp32 MFMA GEMM; ``out``
+    may be res."""
+    _on_gpu(x, weight)
+    for t in (x, weight, bias, res, out):
+        if t is not None and (t.dtype != torch.float32 or t.stride(-1) != 1 or t.device != x.device):
+            raise RuntimeError("gemm_f32: operands must be fp32 with contiguous rows on one device")
+    M, K = x.shape
+    N = weight.shape[0]
+    if weight.shape[1] != K or any(t is not None and t.shape != (M, N) for t in (res, out)) or (bias is not None and bias.shape != (N,)):
+        raise RuntimeError("gemm_f32: x [M, K], weight [N, K], bias [N], res and out [M, N] must match")
+    if out is None:
+        out = torch.empty(M, N, device=x.device, dtype=x.dtype)
+    ev = timer.begin("gemm_f32")
+    _check("hdcm_gemm_f32_fwd", lib().hdcm_gemm_f32_fwd(
+        x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), bias.data_ptr() if bias is not None else None,
+        res.data_ptr() if res is not None else None, res.stride(0) if res is not None else 0, out.data_ptr(), out.stride(0),
+        M, N, K, _stream(x)))
+    timer.end("gemm_f32", ev)
+    return out
+
+
+def gemm_f32_preferred(M, *operands) -> bool:
+    """Whether x weight^T + a bias or residual, of M rows and ``operands`` (x, weight, and the bias or the
+    residual and output), runs on gemm_f32: contiguous aligned fp32 at the sizes of
+    hdcm_gemm_f32_preferred, without recorded library solutions in use."""
+    N, K = operands[1].shape
+    return (all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in operands)
+            and bool(lib().hdcm_gemm_f32_preferred(M, N, K)) and operands[0].shape[-1] == K and not torch.cuda.tunable.is_enabled())
 
 
 def gemm_preferred(x, weight, bias) -> bool:

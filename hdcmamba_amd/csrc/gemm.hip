@@ -44,6 +44,7 @@
 // band), so the workgroups resident on one XCD share a few W and X panels in its L2.
 #include <algorithm>
 
+#include "gemm_tile.h"
 #include "hdcm_common.h"
 
 using namespace hdcm;
@@ -52,35 +53,10 @@ namespace {
 
 constexpr int kBK = 64;
 constexpr int kChunks = kBK / 8;           // 16-byte chunks per tile row
-constexpr int kGroup = 4;                  // o-tiles per band of the workgroup order
-constexpr int kBufferFlags = 0x00020000;   // buffer resource word 3: raw 32-bit dwords
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 enum { EPI_BIAS = 0, EPI_ROWLN = 1, EPI_ROWSTATS = 2 };
 
-// Tile (ot, tt) of this workgroup in the XCD-grouped order above.
-__device__ __forceinline__ void tile_of(int n_otiles, int& ot, int& tt) {
-  const int T = gridDim.x, b = blockIdx.x, x = b & 7, sl = b >> 3;
-  int pre = 0;  // tiles taken by XCDs 0..x-1
-  for (int y = 0; y < x; ++y) pre += (T - y + 7) >> 3;
-  const int i = pre + sl;
-  const int n_tt = T / n_otiles;
-  const int band = i / (kGroup * n_tt), r = i - band * kGroup * n_tt;
-  const int wb = min(kGroup, n_otiles - band * kGroup);
-  tt = r / wb;
-  ot = band * kGroup + (r - tt * wb);
-}
-
-// A workgroup is NWO x NWT waves, a wave NI x NJ MFMA tiles of 16 x 16.
-template <int NWO, int NWT, int NI, int NJ>
-struct Tile {
-  static constexpr int nwo = NWO, nwt = NWT, ni = NI, nj = NJ;
-  static constexpr int BO = NWO * NI * 16, BT = NWT * NJ * 16;
-  static constexpr int waves = NWO * NWT, threads = waves * kWave;
-  static constexpr int WL = BO / waves / 8, XL = BT / waves / 8;  // load instructions per wave and K step
-  static_assert(BO % (waves * 8) == 0 && BT % (waves * 8) == 0 && NI % 2 == 0, "whole 8-row loads, 16-byte runs");
-};
 using Tile256 = Tile<2, 4, 8, 4>;
 using Tile128 = Tile<2, 2, 4, 4>;
 using Tile64 = Tile<2, 2, 2, 2>;
@@ -92,6 +68,7 @@ __global__ __launch_bounds__(TL::threads, TL::threads == 512 ? 1 : 2) void gemm_
     int64_t o_rs, int M, int N, int K, int n_otiles, float eps, const float* __restrict__ wsum,
     const float* __restrict__ rstats, int nparts, int64_t stats_ps) {
   constexpr int kBO = TL::BO, kBT = TL::BT, NI = TL::ni, NJ = TL::nj, NWO = TL::nwo, NWT = TL::nwt;
+  static_assert(NI % 2 == 0, "16-byte runs");
   // four arrays, so that the loads filling one buffer are known not to alias the reads of the other
   __shared__ uint4 sW0[kBO * kChunks], sW1[kBO * kChunks], sX0[kBT * kChunks], sX1[kBT * kChunks];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -435,11 +412,6 @@ __global__ __launch_bounds__(TL::threads, TL::threads == 512 ? 1 : 2) void gemm_
 
 // A workgroup's rows span at most 256 row strides of bytes, addressed with 32-bit offsets.
 bool fits32(int64_t row_stride) { return row_stride <= ((int64_t)1 << 30) / (2 * Tile256::BO); }
-
-template <class TL>
-int64_t tiles_of(int64_t M, int64_t N) {
-  return ((N + TL::BO - 1) / TL::BO) * ((M + TL::BT - 1) / TL::BT);
-}
 
 // Tile width (256, 128 or 64) with the least estimated time, in hundredths of a microsecond.
 // Fitted to measurements: per K step of 64 a 256-wide tile, one workgroup per CU, takes 2.0 us; a

@@ -127,12 +127,26 @@ std::pair<Tensor, Tensor> norm_conv_bwd(const Tensor& go, const Tensor& x, const
   return {dx, dw};
 }
 
+bool aligned(const Tensor& t, size_t n) { return (uintptr_t)t.const_data_ptr() % n == 0; }
+
+// x w^T (+ bias) (+ res) into out, fp32 rows [M, K] and [M, N]
+void gemm_f32(const Tensor& x, const Tensor& w, const float* bias, const float* res, Tensor& out, int64_t M, void* s) {
+  const int64_t K = w.size(1), N = w.size(0);
+  check("hdcm_gemm_f32_fwd", hdcm_gemm_f32_fwd(x.const_data_ptr<float>(), K, w.const_data_ptr<float>(), K, bias, res, N,
+                                               out.mutable_data_ptr<float>(), N, M, N, K, s));
+}
+
 Tensor in_proj(const Tensor& x, const Tensor& w, const Tensor& b, bool library, void* s) {
   const int64_t K = x.size(-1), M = K ? x.numel() / K : 0, N = w.size(0);
-  const auto aligned = [](const Tensor& t, size_t n) { return (uintptr_t)t.const_data_ptr() % n == 0; };
-  if (library || !hdcm_gemm_preferred(M, N, K, dtype_of(x)) || !aligned(x, 16) || !aligned(w, 16) || !aligned(b, 8))
+  const bool f32 = dtype_of(x) == HDCM_F32;
+  if (library || !(f32 ? hdcm_gemm_f32_preferred(M, N, K) : hdcm_gemm_preferred(M, N, K, HDCM_BF16)) ||
+      !aligned(x, 16) || !aligned(w, 16) || !aligned(b, f32 ? 16 : 8))
     return at::linear(x, w, b);
   Tensor out = at::empty({x.size(0), x.size(1), N}, x.options());
+  if (f32) {
+    gemm_f32(x, w, b.const_data_ptr<float>(), nullptr, out, M, s);
+    return out;
+  }
   check("hdcm_gemm_fwd", hdcm_gemm_fwd(x.const_data_ptr(), K, w.const_data_ptr(), K, b.const_data_ptr(),
                                        out.mutable_data_ptr(), N, M, N, K, HDCM_BF16, s));
   return out;
@@ -223,7 +237,10 @@ ForwardOut forward(const Tensor& x, const Params& p, const Dims& d, const Stream
   } else {
     row_norm(m.combined, m.combined, st.main);
     Tensor o2 = out.view({M, dm});
-    if (out.const_data_ptr() == x.const_data_ptr()) o2.addmm_(m.combined.view({M, K}), p.w_out.t());
+    if (dtype_of(x) == HDCM_F32 && !library && hdcm_gemm_f32_preferred(M, dm, K) && aligned(m.combined, 16) &&
+        aligned(p.w_out, 16) && aligned(x, 16) && aligned(out, 16))
+      gemm_f32(m.combined, p.w_out, nullptr, x.const_data_ptr<float>(), o2, M, st.main);
+    else if (out.const_data_ptr() == x.const_data_ptr()) o2.addmm_(m.combined.view({M, K}), p.w_out.t());
     else at::addmm_out(o2, x.view({M, dm}), m.combined.view({M, K}), p.w_out.t());
   }
   return {out, m};
@@ -429,8 +446,7 @@ std::vector<Tensor> norm_conv_backward(const Tensor& go_, const Tensor& x_, cons
 // Weight gradient y^T x of row-major y [M, N], x [M, K] and, with sums, y's column sums
 std::pair<Tensor, Tensor> weight_grad(const Tensor& y, const Tensor& x, bool sums, bool library, void* s) {
   const int64_t M = y.size(0), N = y.size(1), K = x.size(1);
-  const auto aligned = [](const Tensor& t) { return (uintptr_t)t.const_data_ptr() % 16 == 0; };
-  if (library || !hdcm_gemm_tn_preferred(M, N, K, sums, dtype_of(y)) || !aligned(y) || !aligned(x))
+  if (library || !hdcm_gemm_tn_preferred(M, N, K, sums, dtype_of(y)) || !aligned(y, 16) || !aligned(x, 16))
     return {at::mm(y.t(), x), sums ? y.sum(0) : Tensor()};
   Tensor w = at::empty({N, K}, y.options()), c = sums ? at::empty({N}, y.options()) : Tensor();
   const size_t n = hdcm_gemm_tn_workspace_bytes(M, N, K);

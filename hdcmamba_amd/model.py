@@ -23,6 +23,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 from torch.utils.checkpoint import checkpoint
 
 from . import _ops
@@ -277,7 +278,12 @@ class HdcMamba9v3Block(nn.Module):
         x_conv = fused_norm_conv1d_trainable(x, self.norm, self.conv1d)
         w_in, b_in = self.in_proj.weight.to(dtype), self.in_proj.bias.to(dtype)
         # the SSM and slot kernels are constants for autograd, so projs needs no graph either
-        projs = _ops.gemm(x_conv, w_in, b_in) if _ops.gemm_preferred(x_conv, w_in, b_in) else F.linear(x_conv, w_in, b_in)
+        if _ops.gemm_preferred(x_conv, w_in, b_in):
+            projs = _ops.gemm(x_conv, w_in, b_in)
+        elif _ops.gemm_f32_preferred(B * L, x_conv, w_in, b_in):
+            projs = _ops.gemm_f32(x_conv.view(B * L, dm), w_in, b_in).view(B, L, -1)
+        else:
+            projs = F.linear(x_conv, w_in, b_in)
         combined = torch.empty(B, L, ds + dm, device=x.device, dtype=dtype)
         # The SSM and the slot kernels read projs and write disjoint columns of `combined`,
         # so the SSM may run on a side stream beside some of the slot kernels (ssm_overlap:
@@ -359,10 +365,10 @@ class HdcMamba9v3Block(nn.Module):
     # ------------------------------------------------------------------ native host path
     def _native_ok(self, x):
         """Whether the native host path (csrc/native.cpp) takes x: everything but empty inputs, heads
-        wider than the fused slot kernels', launches being timed one by one, and autocast to
-        another dtype; the Python composition below takes the rest, with the same kernels."""
+        wider than the fused slot kernels', launches being timed one by one, autocast to
+        another dtype and forward-mode differentiation; the Python composition below takes the rest, with the same kernels."""
         return (x.dtype in _ops._DTYPES and self.head_dim <= _ops.SLOT_MAX_HEAD_DIM and x.numel() > 0
-                and not _ops.timer.active and self.ssm_overlap in ("auto", "none", "state", "gate", "after_state")
+                and not _ops.timer.active and forward_ad._current_level < 0 and self.ssm_overlap in ("auto", "none", "state", "gate", "after_state")
                 and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype))
 
     def _params(self):
@@ -482,8 +488,14 @@ class HdcMamba9v3Block(nn.Module):
             c = self._differentiable_mixer(x)
         else:
             c = self._mixer(x, state)
-        out = torch.addmm(x.reshape(B * L, dm), c, self.out_proj.weight.to(x.dtype).t())
-        return out.view(B, L, dm)
+        return self._out_proj(x.reshape(B * L, dm), c).view(B, L, dm)
+
+    def _out_proj(self, x, c, out=None):
+        """x + c @ out_proj.weight^T of rows x [M, dm], c [M, ds + dm], into ``out`` (which may be x) when given."""
+        w = self.out_proj.weight.to(x.dtype)
+        if not torch.is_grad_enabled() and forward_ad._current_level < 0 and _ops.gemm_f32_preferred(x.shape[0], c, w, x):
+            return _ops.gemm_f32(c, w, res=x, out=out)
+        return torch.addmm(x, c, w.t()) if out is None else out.addmm_(c, w.t())
 
     def _residual_step_(self, r, state=None):
         """In-place variant for a model-owned residual stream r [B,L,dm] (chunk-aligned):
@@ -495,7 +507,8 @@ class HdcMamba9v3Block(nn.Module):
             self._fused_mixer_out(r, state, out=r)
             return r
         c = self._mixer(r, state)
-        r.view(B * L, dm).addmm_(c, self.out_proj.weight.to(r.dtype).t())
+        r2 = r.view(B * L, dm)
+        self._out_proj(r2, c, out=r2)
         return r
 
     # ------------------------------------------------------------------ prefill / decode

@@ -440,6 +440,18 @@ int hdcm_gemm_fwd(const void* x, int64_t x_row_stride, const void* w, int64_t w_
                   int dtype, void* stream);
 
 /*
+ * Tiled fp32 GEMM: out[t,o] = sum_k x[t,k] w[o,k] (+ bias[o]) (+ res[t,o]) for t < M, o < N in fp32
+ * throughout, sums of 128 products added up in a second accumulator.  bias and res may be NULL; res
+ * may alias out.  Needs K % 4 == 0, N % 4 == 0, 16-byte aligned rows of every operand.  Replaces the
+ * nn.Linear in_proj and out_proj of an fp32 forward (hdcmamba/model.py:313,320).
+ * hdcm_gemm_f32_preferred: whether it is the faster choice against the library's product (1 or 0).
+ */
+int hdcm_gemm_f32_preferred(int64_t M, int64_t N, int64_t K);
+int hdcm_gemm_f32_fwd(const float* x, int64_t x_row_stride, const float* w, int64_t w_row_stride, const float* bias,
+                      const float* res, int64_t res_row_stride, float* out, int64_t out_row_stride, int64_t M,
+                      int64_t N, int64_t K, void* stream);
+
+/*
  * out_proj over the row LayerNorm without affine, with the residual add:
  *   out[t,o] = res[t,o] + r_t * (sum_k c[t,k] w[o,k] - mu_t * s_o),  s_o = sum_k w[o,k]
  * which equals res + LN(c) w^T with LN(c)_t = (c_t - mu_t) r_t over the K columns of row t

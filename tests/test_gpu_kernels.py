@@ -804,6 +804,32 @@ def test_gemm_tile_widths(dev, M, N, K):
         assert (err <= 2 ** -8 * ref.abs() + 2e-3).all(), f"{what}: max err {err.max().item()}"
 
 
+@pytest.mark.parametrize("M,N,K,bias,res", [
+    # one row and 4 columns; 32-wide tiles ragged in rows, columns and K; K steps of 1, 4 (one partial sum),
+    # 5; 64-wide tiles whole and ragged, one and many per CU; the default layer's in_proj and out_proj
+    (1, 4, 4, True, False), (33, 36, 36, True, True), (97, 1216, 256, True, False), (250, 132, 128, False, True),
+    (256, 3264, 768, False, False), (2049, 1028, 132, True, True), (2048, 2240, 512, True, False), (2048, 512, 576, False, True)])
+def test_gemm_f32(dev, M, N, K, bias, res):
+    """The fp32 GEMM against fp64, out aliasing the residual too.  A value is rounded at most 33 times
+    in its partial sum of 128 products, once per partial sum and for the bias and the residual, each by at most
+    2^-24 of the sum of magnitudes; four more for the products themselves."""
+    _say("gemm_f32", M, N, K, bias, res)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    big = torch.randn(M, K + 8, generator=g, device=dev)
+    x = big[:, 4:4 + K]  # strided rows
+    w = torch.randn(N, K, generator=g, device=dev) / K ** 0.5
+    b = torch.randn(N, generator=g, device=dev) if bias else None
+    r = torch.randn(M, N, generator=g, device=dev) if res else None
+    out = _ops.gemm_f32(x, w, b, r)
+    ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    for t in (b, r):
+        if t is not None:
+            ref, mag = ref + t.double(), mag + t.double().abs()
+    assert ((out.double() - ref).abs() <= (40 + K / 128) * 2 ** -24 * mag).all()
+    if res:
+        assert torch.equal(_ops.gemm_f32(x, w, b, r, out=r), out)
+
+
 @pytest.mark.parametrize("M,N,K,sums", [
     # one row, fewer rows than a step, rows not a multiple of the step in the last range, one and many
     # ranges, tiles ragged in both outputs (one group over; less than a tile), more tiles than two per CU

@@ -942,7 +942,7 @@ def gemm_preferred(x, weight, bias) -> bool:
     """Whether linear(x, weight, bias) runs on the tiled GEMM (gemm) rather than the library's:
     bf16 in the layout it takes at the sizes of hdcm_gemm_preferred.  With recorded library
     solutions in use (use_tuned_gemms: in_proj at 32768 rows of d_model 768 162 us, the tiled
-    GEMM 201, the library's default 264) the library keeps all."""
+    GEMM 171, the library's default 265) the library keeps all."""
     K = x.shape[-1]
     return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and bias.dtype == torch.bfloat16
             and bool(lib().hdcm_gemm_preferred(x.numel() // K if K else 0, weight.shape[0], K, HDCM_BF16))

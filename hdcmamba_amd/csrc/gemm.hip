@@ -20,9 +20,11 @@
 // v_mfma_f32_16x16x32_bf16; it moves the fewest LDS and L2 bytes per MFMA.  128: 4 waves of 4 x
 // 4 tiles, 64 KB of LDS, two workgroups per CU covering each other's barriers.  64: 4 waves of
 // 2 x 2 tiles, five workgroups per CU.  W is the MFMA A operand and X is B, so lane l holds
-// outputs of token l % 16 and four consecutive features 4 (l / 16) .. +3 (one 8-byte store).  K advances 64 at a time through two LDS buffers filled by direct-to-LDS buffer
+// outputs of token l % 16 and four consecutive features 4 (l / 16) .. +3; two column tiles are traded between lanes
+// (v_permlane16_swap) into 16-byte stores of 64 bytes a row, where 8-byte ones took 18 of 183 us at
+// 32768 x 3264 x 768.  K advances 64 at a time through two LDS buffers filled by direct-to-LDS buffer
 // loads (buffer_load_dwordx4 ... lds): while tile k feeds the MFMAs, tile k+1 streams into
-// the other buffer; one barrier per K step.  Each load instruction of a wave fills 8 rows
+// the other buffer; one barrier per K step, in EPI_BIAS between the step's halves (188 -> 183 us).  Each load instruction of a wave fills 8 rows
 // x 128 bytes; in LDS the 16-byte chunk c of row r sits at chunk c ^ (r & 7), so the
 // fragment reads of lanes 0..7 (rows r..r+7, one chunk) fall in eight different bank
 // groups (SQ_LDS_BANK_CONFLICT reads 0).  Rows past M or N read as zeros (buffer range
@@ -210,74 +212,114 @@ __global__ __launch_bounds__(TL::threads, TL::threads == 512 ? 1 : 2) void gemm_
   for (int i = 0; i < NI; ++i) wsm[i] = 0.f;
   const bf16x2_t ones = __builtin_bit_cast(bf16x2_t, 0x3f803f80u);
 
-  auto compute = [&](const uint4* bw, const uint4* bx, int kt) {
-    Frag<bf16_t> fa[2][NI], fb[2][NJ];
+  // fragments of K half kk of the tile in bw, bx, and its MFMAs
+  Frag<bf16_t> fa[2][NI], fb[2][NJ];
+  auto read = [&](const uint4* bw, const uint4* bx, int kk) {
+    const int pcf = (kk * 4 + g) ^ (l16 & 7);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int pcf = (kk * 4 + g) ^ (l16 & 7);
+    for (int i = 0; i < NI; ++i)
+      fa[kk][i].v = __builtin_bit_cast(bf16x8_t, bw[(wo0 + i * 16 + l16) * kChunks + pcf]);
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
-        fa[kk][i].v = __builtin_bit_cast(bf16x8_t, bw[(wo0 + i * 16 + l16) * kChunks + pcf]);
+    for (int j = 0; j < NJ; ++j)
+      fb[kk][j].v = __builtin_bit_cast(bf16x8_t, bx[(wt0 + j * 16 + l16) * kChunks + pcf]);
+  };
+  auto compute = [&](int kk) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)
-        fb[kk][j].v = __builtin_bit_cast(bf16x8_t, bx[(wt0 + j * 16 + l16) * kChunks + pcf]);
-    }
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = mma(fa[kk][i], fb[kk][j], acc[i][j]);
-    // the first K half's fragment reads, then the second half's spread over the MFMAs (two
-    // between reads, one in the 64-wide tile, whose halves are four MFMAs each)
-    constexpr int NF = NI + NJ, PER = NI * NJ >= 2 * NF ? 2 : 1;
-    __builtin_amdgcn_sched_group_barrier(0x100, NF, 0);
+      for (int j = 0; j < NJ; ++j) acc[i][j] = mma(fa[kk][i], fb[kk][j], acc[i][j]);
+  };
+  // one half's MFMAs with the other half's fragment reads spread over them, two MFMAs to a read (one in the
+  // 64-wide tile, whose halves are four MFMAs each)
+  constexpr int NF = NI + NJ, PER = NI * NJ >= 2 * NF ? 2 : 1;
+  auto spread = [&] {
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 2 * NI * NJ - PER * NF, 0);
-    if (EPI == EPI_ROWLN) {
-      // after the MFMAs: these need every fragment of the step
-      if (kt % NWO == wo) {
+    __builtin_amdgcn_sched_group_barrier(0x008, NI * NJ - PER * NF, 0);
+  };
+  auto stats = [&](int kk, int kt) {
+    if (EPI != EPI_ROWLN) return;
+    if (kt % NWO == wo) {
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
+      for (int j = 0; j < NJ; ++j) {
+        const uint4 u = __builtin_bit_cast(uint4, fb[kk][j].v);
+        const unsigned d[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) {
-            const uint4 u = __builtin_bit_cast(uint4, fb[kk][j].v);
-            const unsigned d[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const bf16x2_t p = __builtin_bit_cast(bf16x2_t, d[e]);
-              ssum[j] = __builtin_amdgcn_fdot2_f32_bf16(p, ones, ssum[j], false);
-              ssq[j] = __builtin_amdgcn_fdot2_f32_bf16(p, p, ssq[j], false);
-            }
-          }
+        for (int e = 0; e < 4; ++e) {
+          const bf16x2_t p = __builtin_bit_cast(bf16x2_t, d[e]);
+          ssum[j] = __builtin_amdgcn_fdot2_f32_bf16(p, ones, ssum[j], false);
+          ssq[j] = __builtin_amdgcn_fdot2_f32_bf16(p, p, ssq[j], false);
+        }
       }
-      if (kt % NWT == wt) {
+    }
+    if (kt % NWT == wt) {
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
+      for (int i = 0; i < NI; ++i) {
+        const uint4 u = __builtin_bit_cast(uint4, fa[kk][i].v);
+        const unsigned d[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-          for (int i = 0; i < NI; ++i) {
-            const uint4 u = __builtin_bit_cast(uint4, fa[kk][i].v);
-            const unsigned d[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              wsm[i] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, d[e]), ones, wsm[i], false);
-          }
+        for (int e = 0; e < 4; ++e)
+          wsm[i] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, d[e]), ones, wsm[i], false);
       }
     }
   };
 
   const int nk = (K + kBK - 1) / kBK;
-  if constexpr (EPI != EPI_ROWSTATS) issue(sW0, sX0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    const bool odd = kt & 1;
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of tile kt are in LDS
-    __syncthreads();                     // everyone's; and tile kt-1's buffer is free again
-    if (kt + 1 < nk) issue(odd ? sW0 : sW1, odd ? sX0 : sX1, (kt + 1) * kBK);
-    compute(odd ? sW1 : sW0, odd ? sX1 : sX0, kt);
+  if constexpr (EPI == EPI_BIAS) {
+    // A K step's barrier falls between its two halves: the second half's fragments are in registers
+    // by then, so the MFMAs go on while the next step's first fragments are read, and the buffer
+    // just read is free for the loads of the step after it, which have a whole step to land.  With the
+    // other epilogues' registers this order spills (32768 x 1024 x 1152 80 us without it, 100 with).
+    issue(sW0, sX0, 0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of tile 0 are in LDS
+    __syncthreads();                     // everyone's
+    if (nk > 1) issue(sW1, sX1, kBK);
+    read(sW0, sX0, 0);
+    auto step = [&](uint4* bw, uint4* bx, const uint4* next_w, const uint4* next_x, int kt) {
+      read(bw, bx, 1);
+      compute(0);
+      spread();
+      if (kt + 1 < nk) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0070);  // this wave's loads of tile kt + 1 are in LDS, its reads of tile kt done
+        __syncthreads();                     // everyone's
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + 2 < nk) issue(bw, bx, (kt + 2) * kBK);
+        read(next_w, next_x, 0);
+      }
+      compute(1);
+      spread();
+    };
+    for (int kt = 0; kt < nk; kt += 2) {
+      step(sW0, sX0, sW1, sX1, kt);
+      if (kt + 1 < nk) step(sW1, sX1, sW0, sX0, kt + 1);
+    }
+  } else {
+    if constexpr (EPI == EPI_ROWLN) issue(sW0, sX0, 0);
+    for (int kt = 0; kt < nk; ++kt) {
+      const bool odd = kt & 1;
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of tile kt are in LDS
+      __syncthreads();                     // everyone's; and tile kt-1's buffer is free again
+      if (kt + 1 < nk) issue(odd ? sW0 : sW1, odd ? sX0 : sX1, (kt + 1) * kBK);
+      read(odd ? sW1 : sW0, odd ? sX1 : sX0, 0);
+      read(odd ? sW1 : sW0, odd ? sX1 : sX0, 1);
+      compute(0);
+      compute(1);
+      // the first K half's fragment reads, then the second half's spread over the MFMAs
+      __builtin_amdgcn_sched_group_barrier(0x100, NF, 0);
+#pragma unroll
+      for (int r = 0; r < NF; ++r) {
+        __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * NI * NJ - PER * NF, 0);
+      // after the MFMAs: these need every fragment of the step
+      stats(0, kt);
+      stats(1, kt);
+    }
   }
 
   if constexpr (EPI == EPI_ROWSTATS) {
@@ -383,6 +425,31 @@ __global__ __launch_bounds__(TL::threads, TL::threads == 512 ? 1 : 2) void gemm_
       cst[i][0] = cst[i][1] = cst[i][2] = cst[i][3] = 0.f;
     }
   }
+  if constexpr (EPI == EPI_BIAS) {
+    if (N % 8 == 0 && o_rs % 8 == 0 && ((uintptr_t)out & 15u) == 0) {  // 16-byte runs, as EPI_ROWSTATS writes them
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int t = t0 + wt0 + j * 16 + l16;
+#pragma unroll
+        for (int ip = 0; ip < NI / 2; ++ip) {
+          uint32_t w2[2][2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int i = 2 * ip + h;
+            const f32x4_t a = acc[i][j];
+            w2[h][0] = pack_bf16x2(a[0] + cst[i][0], a[1] + cst[i][1]);
+            w2[h][1] = pack_bf16x2(a[2] + cst[i][2], a[3] + cst[i][3]);
+          }
+          const auto s0 = __builtin_amdgcn_permlane16_swap(w2[0][0], w2[1][0], false, false);
+          const auto s1 = __builtin_amdgcn_permlane16_swap(w2[0][1], w2[1][1], false, false);
+          const int o = o0 + wo0 + ip * 32 + gcol;
+          if (t < M && o < N)
+            *reinterpret_cast<uint4*>(out + (int64_t)t * o_rs + o) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+        }
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     if (EPI == EPI_ROWLN && j + 1 < NJ) load_res(j + 1, rnext);
@@ -421,7 +488,8 @@ bool fits32(int64_t row_stride) { return row_stride <= ((int64_t)1 << 30) / (2 *
 // K loop.  Out_proj with the folded LayerNorm at K = 832, N = 768: 4096 rows 28.4 us with 256,
 // 14.0 with 128, 12.4 with 64; 8192 rows 29.4, 18.9, 21.8; 32768 rows 70.6, 67.8, 91.3.  In_proj
 // at K = 768, N = 3264: 2048 rows 27.6, 17.4, 21.0; 8192 rows 54.9, 58.5, 71.6; 32768 rows 201,
-// 213, 292.  K = 1024, N = 4480, 32768 rows: 318, 358, 471.
+// 213, 292.  K = 1024, N = 4480, 32768 rows: 318, 358, 471 (in_proj's before its wider stores, which gave the
+// 256-wide tile 171 and 273 at 32768 rows and left the order of the widths).
 int tile_choice(int64_t M, int64_t N, int64_t K) {
   const int64_t kCus = 256, nk = (K + kBK - 1) / kBK;
   const auto per_cu = [&](int64_t tiles) { return (tiles + kCus - 1) / kCus; };
@@ -488,12 +556,13 @@ extern "C" int hdcm_gemm_fwd(const void* x, int64_t x_row_stride, const void* w,
             0, (hipStream_t)stream);
 }
 
-// K <= 768 and at most 32768 rows: there the library's default solution measured slower (in_proj, N
-// = 4 K + 192: K 768, 32768 rows 264 against 201 us, 8192 rows 70 against 55; K 512, 8192 rows 39
-// against 32; K 256, 16384 rows 34 against 23); at K 1024, 32768 rows it is 255 against 318 us, at K
-// 512, 131072 rows 387 against 459.
+// Where the library's default solution measured slower (in_proj, N = 4 K + 192 or 4 K + 384; us, library and
+// this): K 768, 32768 rows 265, 171; 8192 rows 70, 49; K 256, 16384 rows 34, 24; K 1024, 16384 rows
+// 161, 150; 1024 rows 19.2, 18.6.  Beyond it is as fast or faster: K 768, 65536 rows 314, 336; K 1024,
+// 32768 rows 251, 273; K 512, 131072 rows 376, 397; K 1536, 8192 rows 154, 161; K 2048, 16128 rows 419, 469.
 extern "C" int hdcm_gemm_preferred(int64_t M, int64_t N, int64_t K, int dtype) {
-  return dtype == HDCM_BF16 && K > 0 && K <= 768 && K % 8 == 0 && N > 0 && N % 4 == 0 && M > 0 && M <= 32768;
+  return dtype == HDCM_BF16 && K > 0 && K <= 1024 && K % 8 == 0 && N > 0 && N % 4 == 0 && M > 0 &&
+         M <= (K <= 768 ? 32768 : 16384);
 }
 
 extern "C" int hdcm_rowln_gemm_fwd(const void* c, int64_t c_row_stride, const void* w, int64_t w_row_stride,

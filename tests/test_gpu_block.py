@@ -316,6 +316,7 @@ def _composition(blk):
     (torch.bfloat16, 256, 64, 4, 64, 3, 100),   # padded
     (torch.bfloat16, 64, 8, 2, 8, 1, 13),       # at most 16 rows: statistics inside the GEMM
     (torch.bfloat16, 100 * 8, 32, 10, 64, 1, 65),  # d_model 800: in_proj on the library GEMM
+    (torch.bfloat16, 17 * 64, 32, 17, 64, 1, 65),  # d_model 1088: past the tiled GEMM's sizes
     (torch.float32, 256, 64, 8, 64, 2, 100), (torch.float32, 48, 12, 1, 20, 1, 20)])
 def test_native_forward_is_the_composition(dev, dtype, dm, ds, H, C, B, L):
     """The native host path issues the composition's kernels on the same operands: forward,

@@ -109,6 +109,10 @@ _PROTOS = {
     "hdcm_norm_conv_bwd": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
                                    c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
                                    c_void_p, c_size_t, c_int64, c_int64, c_int64, c_float, c_int, c_void_p]),
+    "hdcm_norm_conv_bwd_add": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
+                                       c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,
+                                       c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_int64, c_int64, c_int64,
+                                       c_float, c_int, c_void_p]),
 }
 
 _lib = None
@@ -367,9 +371,9 @@ def norm_conv(x, ln_w, ln_b, conv_w, conv_b, eps, out=None):
     return out
 
 
-def norm_conv_bwd(grad_out, x, ln_w, ln_b, conv_w, eps):
-    """Gradients of norm_conv: returns dx (x.dtype, [B,L,D]) and fp32 d_ln_w [D],
-    d_ln_b [D], d_conv_w [D,4], d_conv_b [D]."""
+def norm_conv_bwd(grad_out, x, ln_w, ln_b, conv_w, eps, res=None):
+    """Gradients of norm_conv: returns dx (x.dtype, [B,L,D]; plus ``res`` [B,L,D], unit inner stride, when
+    given) and fp32 d_ln_w [D], d_ln_b [D], d_conv_w [D,4], d_conv_b [D]."""
     _on_gpu(grad_out, x)
     B, L, D = x.shape
     ln_w = _same(ln_w, x, "ln_w")
@@ -386,9 +390,12 @@ def norm_conv_bwd(grad_out, x, ln_w, ln_b, conv_w, eps):
     d_conv_w = torch.empty(D, 4, **f32)
     nbytes = lib().hdcm_norm_conv_bwd_workspace_bytes(B, L, D)
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
-    _check("hdcm_norm_conv_bwd", lib().hdcm_norm_conv_bwd(
+    if res is not None and (res.shape != x.shape or res.dtype != x.dtype or res.device != x.device or res.stride(2) != 1):
+        raise RuntimeError("norm_conv_bwd: res must match x, with a contiguous last dimension")
+    r = (res.data_ptr(), res.stride(0), res.stride(1)) if res is not None else (None, 0, 0)
+    _check("hdcm_norm_conv_bwd_add", lib().hdcm_norm_conv_bwd_add(
         grad_out.data_ptr(), grad_out.stride(0), grad_out.stride(1), x.data_ptr(), x.stride(0), x.stride(1),
-        ln_w.data_ptr(), ln_b.data_ptr(), conv_w.data_ptr(), dx.data_ptr(), dx.stride(0), dx.stride(1),
+        ln_w.data_ptr(), ln_b.data_ptr(), conv_w.data_ptr(), *r, dx.data_ptr(), dx.stride(0), dx.stride(1),
         d_ln_w.data_ptr(), d_ln_b.data_ptr(), d_conv_w.data_ptr(), d_conv_b.data_ptr(), ws.data_ptr(), nbytes,
         B, L, D, float(eps), _dtype(x), _stream(x)))
     return dx, d_ln_w, d_ln_b, d_conv_w, d_conv_b

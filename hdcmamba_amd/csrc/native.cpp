@@ -110,18 +110,20 @@ Tensor norm_conv(const Tensor& x, const Tensor& nw, const Tensor& nb, const Tens
   return out;
 }
 
-// dx (x's dtype) and, as one fp32 buffer [7 D], d norm w, d norm b, d conv w [D, 4], d conv b
+// dx (x's dtype; with res [B, L, D] contiguous, plus res) and, as one fp32 buffer [7 D], d norm w, d norm b,
+// d conv w [D, 4], d conv b
 std::pair<Tensor, Tensor> norm_conv_bwd(const Tensor& go, const Tensor& x, const Tensor& nw, const Tensor& nb, const Tensor& cw,
-                                  double eps, void* s) {
+                                  const Tensor* res, double eps, void* s) {
   const int64_t B = x.size(0), L = x.size(1), D = x.size(2);
   Tensor dx = at::empty({B, L, D}, x.options());
   Tensor dw = fp32({7 * D}, x);
   float* p = dw.mutable_data_ptr<float>();
   const size_t n = hdcm_norm_conv_bwd_workspace_bytes(B, L, D);
   Tensor ws = bytes(n, x);
-  check("hdcm_norm_conv_bwd",
-        hdcm_norm_conv_bwd(go.const_data_ptr(), go.stride(0), go.stride(1), x.const_data_ptr(), x.stride(0), x.stride(1),
-                           nw.const_data_ptr(), nb.const_data_ptr(), cw.const_data_ptr(), dx.mutable_data_ptr(),
+  check("hdcm_norm_conv_bwd_add",
+        hdcm_norm_conv_bwd_add(go.const_data_ptr(), go.stride(0), go.stride(1), x.const_data_ptr(), x.stride(0), x.stride(1),
+                           nw.const_data_ptr(), nb.const_data_ptr(), cw.const_data_ptr(), res ? res->const_data_ptr() : nullptr,
+                           L * D, D, dx.mutable_data_ptr(),
                            dx.stride(0), dx.stride(1), p, p + D, p + 2 * D, p + 6 * D, ws.mutable_data_ptr(), n, B, L, D,
                            (float)eps, dtype_of(x), s));
   return {dx, dw};
@@ -438,7 +440,7 @@ std::vector<Tensor> norm_conv_backward(const Tensor& go_, const Tensor& x_, cons
   const Tensor x = x_.stride(2) == 1 ? x_ : x_.contiguous();
   const int64_t D = x.size(2);
   auto g = norm_conv_bwd(same(go_, x, "grad_out"), x, same(nw, x, "ln_w"), same(nb, x, "ln_b"),
-                         same(cw.reshape({D, 4}), x, "conv_w"), eps, (void*)stream);
+                         same(cw.reshape({D, 4}), x, "conv_w"), nullptr, eps, (void*)stream);
   const Tensor w = g.second.to(x.scalar_type());
   return {g.first, w.narrow(0, 0, D), w.narrow(0, D, D), w.narrow(0, 2 * D, 4 * D).view(cw.sizes()), w.narrow(0, 6 * D, D)};
 }
@@ -520,8 +522,9 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
   }
   if (need[0] || need[1] || need[2] || need[3] || need[4]) {
     Tensor dxc = at::mm(dproj2, p.w_in).view({B, L, dm});
-    auto n = norm_conv_bwd(dxc, x, p.nw, p.nb, p.cw, p.eps, st.main);
-    if (need[0]) out[0] = n.first.add_(dy);
+    const bool add = aligned(dy, 16);
+    auto n = norm_conv_bwd(dxc, x, p.nw, p.nb, p.cw, add ? &dy : nullptr, p.eps, st.main);
+    if (need[0]) out[0] = add ? n.first : n.first.add_(dy);
     const Tensor w = n.second.to(params[0].scalar_type());
     give(0, w.narrow(0, 0, dm));
     give(1, w.narrow(0, dm, dm));

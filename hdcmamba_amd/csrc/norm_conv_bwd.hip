@@ -41,47 +41,35 @@ template <typename T, int NG, int WPR>
 __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_conv_bwd_kernel(
     const T* __restrict__ go, int64_t g_bs, int64_t g_rs, const T* __restrict__ x, int64_t x_bs, int64_t x_rs,
     const T* __restrict__ ln_w, const T* __restrict__ conv_w, T* __restrict__ dx, int64_t d_bs, int64_t d_rs,
-    float* __restrict__ part, int L, int D, float eps, int run_rows, int runs_per_seq, int nruns) {
+    const T* __restrict__ res, int64_t r_bs, int64_t r_rs, float* __restrict__ part, int L, int D, float eps, int run_rows, int runs_per_seq, int nruns) {
   constexpr int E = Vec<T>::N;
   constexpr int CW = WPR * kWave;   // column lanes of a row
   constexpr int SL = kWpb / WPR;    // runs of a workgroup
   constexpr int W = NG * CW * E;    // columns those lanes span
-  __shared__ float red[2][kWpb][2];
+  __shared__ __attribute__((aligned(16))) float red[2][kWpb][4];
   __shared__ __attribute__((aligned(16))) float cols[SL > 1 ? 5 * W : 4];
   const int wave = threadIdx.x / kWave, slice = wave / WPR;
   const int lane = threadIdx.x % CW;  // column lane
   const int run = (int)blockIdx.x * SL + slice;
   const int G = D / E;
-  // Row totals of one or two values: within the wave, then (WPR > 1) across the waves through
-  // LDS.  Two buffers used in turn: a buffer is written again only two reductions later, after
-  // the barrier of the reduction between, which every thread passes after reading it.
+  // Row totals of four values: within the wave, then (WPR > 1) across the waves through LDS.  Two
+  // buffers used in turn: a buffer is written again only two reductions later, after the barrier
+  // of the reduction between, which every thread passes after reading it.
   int parity = 0;
-  auto row_total2 = [&](float& a, float& c) {
-    a = wave_total(a);
-    c = wave_total(c);
+  auto row_totals = [&](float4 v) {
+    v = make_float4(wave_total(v.x), wave_total(v.y), wave_total(v.z), wave_total(v.w));
     if constexpr (WPR > 1) {
-      if ((threadIdx.x & (kWave - 1)) == 0) {
-        red[parity][wave][0] = a;
-        red[parity][wave][1] = c;
-      }
+      if ((threadIdx.x & (kWave - 1)) == 0) *reinterpret_cast<float4*>(red[parity][wave]) = v;
       __syncthreads();
-      a = c = 0.f;
+      v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int k = 0; k < WPR; ++k) {
-        a += red[parity][slice * WPR + k][0];
-        c += red[parity][slice * WPR + k][1];
+        const float4 u = *reinterpret_cast<const float4*>(red[parity][slice * WPR + k]);
+        v = make_float4(v.x + u.x, v.y + u.y, v.z + u.z, v.w + u.w);
       }
       parity ^= 1;
     }
-  };
-  auto row_total = [&](float a) {
-    if constexpr (WPR > 1) {
-      float c = 0.f;
-      row_total2(a, c);
-      return a;
-    } else {
-      return wave_total(a);
-    }
+    return v;
   };
 
   float X[4][NG][E], Gs[NG][E];
@@ -101,6 +89,7 @@ __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_
   const T* gb = go + (int64_t)b * g_bs;
   const T* xb = x + (int64_t)b * x_bs;
   T* db = dx + (int64_t)b * d_bs;
+  const T* rb = res ? res + (int64_t)b * r_bs : nullptr;
   // raw 16-byte groups of one row; rows past the sequence read its last row (used as zeros)
   auto fetch = [&](uint4 (&v)[NG], const T* base, int64_t rs, int t) {
     const T* row = base + (int64_t)min(t, L - 1) * rs;
@@ -110,15 +99,43 @@ __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_
   bool own[NG];
 #pragma unroll
   for (int i = 0; i < NG; ++i) own[i] = lane + CW * i < G;
-  // g0..g3 = go[t .. t+3]; gn = go[t+4] and xn = x[t+1] are in flight or landed, ga and xa the rows after them
-  uint4 g0[NG], g1[NG], g2[NG], g3[NG], gn[NG], x0[NG], xn[NG];
+  // sum of a row, and of its squared distances from the mean
+  auto sum_of = [&](const uint4 (&raw)[NG]) {
+    float v[E], s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      unpack16<T>(raw[i], v);
+#pragma unroll
+      for (int e = 0; e < E; ++e) s += own[i] ? v[e] : 0.f;
+    }
+    return s;
+  };
+  auto squares_of = [&](const uint4 (&raw)[NG], float mean) {
+    float v[E], q = 0.f;
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      unpack16<T>(raw[i], v);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const float c = own[i] ? v[e] - mean : 0.f;
+        q += c * c;
+      }
+    }
+    return q;
+  };
+  // g0..g3 = go[t .. t+3], x0..x2 = x[t .. t+2]; gn = go[t+4] and xn = x[t+3] are in flight or landed, ga
+  // and xa the rows after them; r0 = res[t]
+  uint4 g0[NG], g1[NG], g2[NG], g3[NG], gn[NG], x0[NG], x1[NG], x2[NG], xn[NG], r0[NG];
+  fetch(x0, xb, x_rs, t0);
+  fetch(x1, xb, x_rs, t0 + 1);
   fetch(g0, gb, g_rs, t0);
   fetch(g1, gb, g_rs, t0 + 1);
   fetch(g2, gb, g_rs, t0 + 2);
   fetch(g3, gb, g_rs, t0 + 3);
+  fetch(x2, xb, x_rs, t0 + 2);
   fetch(gn, gb, g_rs, t0 + 4);
-  fetch(x0, xb, x_rs, t0);
-  fetch(xn, xb, x_rs, t0 + 1);
+  fetch(xn, xb, x_rs, t0 + 3);
+  if (rb) fetch(r0, rb, r_rs, t0);
   float gw[NG][E], cw[4][NG][E];
 #pragma unroll
   for (int i = 0; i < NG; ++i) {
@@ -132,32 +149,29 @@ __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_
 #pragma unroll
       for (int k = 0; k < 4; ++k) cw[k][i][e] = c4[4 * e + k];
   }
+  // A row's reductions (mean, variance, the two gradient sums) form a chain, so each step takes one
+  // round for three rows: the gradient sums of t, the variance of t + 1 and the mean of t + 2.
+  float mean, mean1, rstd;
+  {
+    const float4 m = row_totals(make_float4(sum_of(x0), sum_of(x1), 0.f, 0.f));
+    mean = m.x * invD, mean1 = m.y * invD;
+    rstd = rsqrtf(row_totals(make_float4(squares_of(x0, mean), 0.f, 0.f, 0.f)).x * invD + eps);
+  }
   const int t_end = WPR > 1 ? t0 + run_rows : t1;
 #pragma unroll 1
   for (int t = t0; t < t_end; ++t) {
-    uint4 ga[NG], xa[NG];
+    uint4 ga[NG], xa[NG], ra[NG];
     fetch(ga, gb, g_rs, t + 5);
-    fetch(xa, xb, x_rs, t + 2);
+    fetch(xa, xb, x_rs, t + 4);
+    if (rb) fetch(ra, rb, r_rs, t + 1);
     const bool in_run = t < t1;
     float xv[NG][E], gh[NG][E];
-    float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
       unpack16<T>(x0[i], xv[i]);
 #pragma unroll
-      for (int e = 0; e < E; ++e) s += own[i] ? xv[i][e] : 0.f;
+      for (int e = 0; e < E; ++e) xv[i][e] = own[i] ? xv[i][e] - mean : 0.f;
     }
-    const float mean = row_total(s) * invD;
-    float q = 0.f;
-#pragma unroll
-    for (int i = 0; i < NG; ++i)
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const float c = own[i] ? xv[i][e] - mean : 0.f;
-        xv[i][e] = c;
-        q += c * c;
-      }
-    const float rstd = rsqrtf(row_total(q) * invD + eps);
     const float rx = in_run ? rstd : 0.f;
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
@@ -193,17 +207,26 @@ __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_
         s2 += gh[i][e] * xv[i][e];
       }
     }
-    row_total2(s1, s2);
-    const float m1 = s1 * invD, m2 = s2 * invD;
+    const float4 tot = row_totals(make_float4(s1, s2, squares_of(x1, mean1), sum_of(x2)));
+    const float m1 = tot.x * invD, m2 = tot.y * invD;
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
       float o[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) o[e] = rstd * (gh[i][e] - m1 - xv[i][e] * m2);
+      if (rb) {
+        float rv[E];
+        unpack16<T>(r0[i], rv);
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] += rv[e];
+        r0[i] = ra[i];
+      }
       if (own[i] && in_run) store16<T>(db + (int64_t)t * d_rs + (int64_t)(lane + CW * i) * E, o);
       g0[i] = g1[i], g1[i] = g2[i], g2[i] = g3[i], g3[i] = gn[i], gn[i] = ga[i];
-      x0[i] = xn[i], xn[i] = xa[i];
+      x0[i] = x1[i], x1[i] = x2[i], x2[i] = xn[i], xn[i] = xa[i];
     }
+    mean = mean1, mean1 = tot.w * invD;
+    rstd = rsqrtf(tot.z * invD + eps);
   }
 
   // this workgroup's sums: part[block][5][D] (X_0 .. X_3, G)
@@ -305,7 +328,7 @@ Plan plan_of(int64_t B, int64_t L, int64_t D) {
 template <typename T>
 int launch_bwd(const void* go, int64_t g_bs, int64_t g_rs, const void* x, int64_t x_bs, int64_t x_rs,
                const void* ln_w, const void* ln_b, const void* conv_w, void* dx, int64_t d_bs, int64_t d_rs,
-               float* d_ln_w, float* d_ln_b, float* d_conv_w, float* d_conv_b, void* ws, int64_t B, int64_t L,
+               const void* res, int64_t r_bs, int64_t r_rs, float* d_ln_w, float* d_ln_b, float* d_conv_w, float* d_conv_b, void* ws, int64_t B, int64_t L,
                int64_t D, float eps, hipStream_t s) {
   constexpr int E = Vec<T>::N;
   const int G = (int)(D / E);
@@ -317,7 +340,8 @@ int launch_bwd(const void* go, int64_t g_bs, int64_t g_rs, const void* x, int64_
 #define HDCM_BWD(N, WPR)                                                                                               \
   if (!launched && p.wpr == WPR && ng <= N) {                                                                          \
     HDCM_LAUNCH((norm_conv_bwd_kernel<T, N, WPR>), dim3((unsigned)p.grid), dim3(kWpb * kWave), 0, s, (const T*)go,     \
-                g_bs, g_rs, (const T*)x, x_bs, x_rs, (const T*)ln_w, (const T*)conv_w, (T*)dx, d_bs, d_rs, (float*)ws, \
+                g_bs, g_rs, (const T*)x, x_bs, x_rs, (const T*)ln_w, (const T*)conv_w, (T*)dx, d_bs, d_rs,              \
+                (const T*)res, r_bs, r_rs, (float*)ws,                                                                 \
                 (int)L, (int)D, eps, p.run_rows, p.runs_per_seq, p.nruns);                                             \
     launched = true;                                                                                                   \
   }
@@ -353,12 +377,13 @@ extern "C" size_t hdcm_norm_conv_bwd_workspace_bytes(int64_t B, int64_t L, int64
   return std::max(asked, (size_t)plan_of(B, L, D).grid * 5 * D * sizeof(float));
 }
 
-extern "C" int hdcm_norm_conv_bwd(const void* grad_out, int64_t g_batch_stride, int64_t g_row_stride,
-                                  const void* x, int64_t x_batch_stride, int64_t x_row_stride, const void* ln_w,
-                                  const void* ln_b, const void* conv_w, void* dx, int64_t dx_batch_stride,
-                                  int64_t dx_row_stride, float* d_ln_w, float* d_ln_b, float* d_conv_w,
-                                  float* d_conv_b, void* ws, size_t ws_bytes, int64_t B, int64_t L, int64_t D,
-                                  float eps, int dtype, void* stream) {
+extern "C" int hdcm_norm_conv_bwd_add(const void* grad_out, int64_t g_batch_stride, int64_t g_row_stride,
+                                      const void* x, int64_t x_batch_stride, int64_t x_row_stride, const void* ln_w,
+                                      const void* ln_b, const void* conv_w, const void* res, int64_t res_batch_stride,
+                                      int64_t res_row_stride, void* dx, int64_t dx_batch_stride,
+                                      int64_t dx_row_stride, float* d_ln_w, float* d_ln_b, float* d_conv_w,
+                                      float* d_conv_b, void* ws, size_t ws_bytes, int64_t B, int64_t L, int64_t D,
+                                      float eps, int dtype, void* stream) {
   HDCM_CHECK_ARG(dtype == HDCM_F32 || dtype == HDCM_BF16, HDCM_EUNSUPPORTED);
   HDCM_CHECK_ARG(ln_w && ln_b && conv_w && d_ln_w && d_ln_b && d_conv_w && d_conv_b &&
                      ((grad_out && x && dx) || B == 0 || L == 0),
@@ -371,9 +396,9 @@ extern "C" int hdcm_norm_conv_bwd(const void* grad_out, int64_t g_batch_stride, 
   HDCM_CHECK_ARG(hdcm_aligned16(ln_w) && hdcm_aligned16(ln_b) && hdcm_aligned16(conv_w), HDCM_EALIGN);
   if (B == 0 || L == 0) {  // no rows (strides unused): the parameter gradients are zero
     if (dtype == HDCM_F32)
-      return launch_bwd<float>(nullptr, 0, 0, nullptr, 0, 0, ln_w, ln_b, conv_w, nullptr, 0, 0, d_ln_w, d_ln_b, d_conv_w,
+      return launch_bwd<float>(nullptr, 0, 0, nullptr, 0, 0, ln_w, ln_b, conv_w, nullptr, 0, 0, nullptr, 0, 0, d_ln_w, d_ln_b, d_conv_w,
                                d_conv_b, nullptr, 0, 0, D, eps, (hipStream_t)stream);
-    return launch_bwd<bf16_t>(nullptr, 0, 0, nullptr, 0, 0, ln_w, ln_b, conv_w, nullptr, 0, 0, d_ln_w, d_ln_b, d_conv_w,
+    return launch_bwd<bf16_t>(nullptr, 0, 0, nullptr, 0, 0, ln_w, ln_b, conv_w, nullptr, 0, 0, nullptr, 0, 0, d_ln_w, d_ln_b, d_conv_w,
                               d_conv_b, nullptr, 0, 0, D, eps, (hipStream_t)stream);
   }
   HDCM_CHECK_ARG(g_row_stride >= D && x_row_stride >= D && dx_row_stride >= D, HDCM_EINVAL);
@@ -383,14 +408,27 @@ extern "C" int hdcm_norm_conv_bwd(const void* grad_out, int64_t g_batch_stride, 
   HDCM_CHECK_ARG(hdcm_aligned16(grad_out) && hdcm_aligned16(x) && hdcm_aligned16(dx) && hdcm_aligned16(ln_w) &&
                      hdcm_aligned16(ln_b) && hdcm_aligned16(conv_w),
                  HDCM_EALIGN);
+  HDCM_CHECK_ARG(!res || res_row_stride >= D, HDCM_EINVAL);
+  HDCM_CHECK_ARG(!res || (res_row_stride % E == 0 && res_batch_stride % E == 0 && hdcm_aligned16(res)), HDCM_EALIGN);
   HDCM_CHECK_ARG(ws != nullptr && ws_bytes >= hdcm_norm_conv_bwd_workspace_bytes(B, L, D), HDCM_EWORKSPACE);
   HDCM_CHECK_ARG(((uintptr_t)ws & 255u) == 0, HDCM_EALIGN);
   hipStream_t s = (hipStream_t)stream;
   if (dtype == HDCM_F32)
     return launch_bwd<float>(grad_out, g_batch_stride, g_row_stride, x, x_batch_stride, x_row_stride, ln_w, ln_b,
-                             conv_w, dx, dx_batch_stride, dx_row_stride, d_ln_w, d_ln_b, d_conv_w, d_conv_b, ws, B,
-                             L, D, eps, s);
+                             conv_w, dx, dx_batch_stride, dx_row_stride, res, res_batch_stride, res_row_stride, d_ln_w, d_ln_b,
+                             d_conv_w, d_conv_b, ws, B, L, D, eps, s);
   return launch_bwd<bf16_t>(grad_out, g_batch_stride, g_row_stride, x, x_batch_stride, x_row_stride, ln_w, ln_b,
-                            conv_w, dx, dx_batch_stride, dx_row_stride, d_ln_w, d_ln_b, d_conv_w, d_conv_b, ws, B, L,
-                            D, eps, s);
+                            conv_w, dx, dx_batch_stride, dx_row_stride, res, res_batch_stride, res_row_stride, d_ln_w, d_ln_b,
+                            d_conv_w, d_conv_b, ws, B, L, D, eps, s);
+}
+
+extern "C" int hdcm_norm_conv_bwd(const void* grad_out, int64_t g_batch_stride, int64_t g_row_stride,
+                                  const void* x, int64_t x_batch_stride, int64_t x_row_stride, const void* ln_w,
+                                  const void* ln_b, const void* conv_w, void* dx, int64_t dx_batch_stride,
+                                  int64_t dx_row_stride, float* d_ln_w, float* d_ln_b, float* d_conv_w,
+                                  float* d_conv_b, void* ws, size_t ws_bytes, int64_t B, int64_t L, int64_t D,
+                                  float eps, int dtype, void* stream) {
+  return hdcm_norm_conv_bwd_add(grad_out, g_batch_stride, g_row_stride, x, x_batch_stride, x_row_stride, ln_w, ln_b,
+                                conv_w, nullptr, 0, 0, dx, dx_batch_stride, dx_row_stride, d_ln_w, d_ln_b, d_conv_w,
+                                d_conv_b, ws, ws_bytes, B, L, D, eps, dtype, stream);
 }

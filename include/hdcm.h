@@ -135,6 +135,13 @@ int hdcm_norm_conv_bwd(const void* grad_out, int64_t g_batch_stride, int64_t g_r
                        int64_t dx_row_stride, float* d_ln_w, float* d_ln_b, float* d_conv_w,
                        float* d_conv_b, void* ws, size_t ws_bytes, int64_t B, int64_t L, int64_t D,
                        float eps, int dtype, void* stream);
+/* The same with dx += res [B,L,D] (strides as x), in fp32 before dx is rounded; res NULL adds nothing. */
+int hdcm_norm_conv_bwd_add(const void* grad_out, int64_t g_batch_stride, int64_t g_row_stride,
+                       const void* x, int64_t x_batch_stride, int64_t x_row_stride, const void* ln_w,
+                       const void* ln_b, const void* conv_w, const void* res, int64_t res_batch_stride, int64_t res_row_stride, void* dx, int64_t dx_batch_stride,
+                       int64_t dx_row_stride, float* d_ln_w, float* d_ln_b, float* d_conv_w,
+                       float* d_conv_b, void* ws, size_t ws_bytes, int64_t B, int64_t L, int64_t D,
+                       float eps, int dtype, void* stream);
 
 /*
  * Diagonal selective scan over ds channels.  For row (b,t) of projs, columns

@@ -88,6 +88,24 @@ def test_norm_conv_backward_runs(dev, dtype, B, L, D):
         assert max_rel(a, e) <= 1e-4, (name, max_rel(a, e))
 
 
+@pytest.mark.parametrize("dtype,B,L,D", [(torch.bfloat16, 2, 1, 256), (torch.bfloat16, 3, 37, 1024), (torch.bfloat16, 1, 130, 2048),
+                                         (torch.float32, 2, 2, 128), (torch.float32, 1, 67, 768), (torch.float32, 1, 35, 3072)])
+def test_norm_conv_backward_add(dev, dtype, B, L, D):
+    """dx with a residual gradient added (runs of one and two rows, one, two and four waves per row): the sum
+    of the two, dx unrounded; the parameter gradients are the same.  A rounding to bf16 is within 2^-8 of
+    the value (8 significant bits): dx's own and the sum's, 2^-7 of |dx| + |res|; fp32 2^-24 each."""
+    _say("norm_conv_bwd add", dtype, B, L, D)
+    g = torch.Generator(device=dev).manual_seed(L + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(dtype)  # noqa: E731
+    x, go, res = rnd(B, L, D), rnd(B, L, D), rnd(B, L, 2 * D)[..., D:]
+    w, b, cw = rnd(D), rnd(D), rnd(D, 1, 4)
+    dx, *dp = _ops.norm_conv_bwd(go, x, w, b, cw, 1e-5)
+    ax, *ap = _ops.norm_conv_bwd(go, x, w, b, cw, 1e-5, res)
+    mag = dx.double().abs() + res.double().abs()
+    assert ((ax.double() - dx.double() - res.double()).abs() <= (2 ** -7 if dtype == torch.bfloat16 else 2 ** -23) * mag).all()
+    assert all(torch.equal(p, q) for p, q in zip(dp, ap))
+
+
 def test_norm_conv_batch_strided(dev):
     """A batch-strided view (rows 3.. of a longer buffer) is read through its strides."""
     g = torch.Generator().manual_seed(7)

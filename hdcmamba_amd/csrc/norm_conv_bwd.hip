@@ -15,17 +15,20 @@
 // by the pass that computes dx: x and go are read once.
 //
 // norm_conv_bwd_kernel: WPR waves (1, 2 or 4) walk a run of rows, lanes owning 16-byte column
-// groups (as the forward) with their five sums and four taps in registers; the rows two ahead are
-// in flight.  Eight columns per lane leave room for two waves per SIMD, so rows take one wave
+// groups (as the forward) with their five sums and four taps in registers; rows come through rings (each go
+// row unpacked once, nothing moved between steps), the next ones in flight.  Eight columns per lane leave room for two waves per SIMD, so rows take one wave
 // up to 512 columns, two up to 1024 and four beyond (row sums then finish across the waves in
 // LDS), up to the forward's 768 groups per row.  Runs are sized for about 2048 waves.  Each
 // workgroup leaves one row of sums [5][D]; norm_conv_bwd_sum_kernel adds them in a fixed order
 // (the result does not depend on scheduling) and forms the gradients.
-// Bound: HBM (x, go read, dx written; go 3 rows more per run).  Measured with the sums, bf16 /
-// fp32: 8 x 4095 rows of 1024 69 / 97 us (2.9 / 4.1 TB/s of that traffic), 135 / 164 us as two
-// passes (dx, then the parameter sums) and three column-sum launches; 4 x 2048 x 768 32 / 31
-// against 88 / 58; 32768 x 256 33 / 32 against 89 / 85.
+// dx may take the gradient of the residual branch with it (res), in place of an addition of its own (23 us at
+// 32768 x 768, bf16).
+// Bound: the vector ALU (about 40 operations a value), then HBM (x, go read, dx written; go 3 rows more per
+// run).  This kernel alone, bf16 8 x 4095 rows of 1024: 50 us, 4.0 TB/s of that traffic; 60 with three chained
+// reductions a row, 56 with one and registers moved every row; fp32 2 x 1024 x 512 18, 20, 17 us.
+// The sums' launch adds 8 us there; two passes (dx, then the sums) and three launches were 135 in all.
 #include <algorithm>
+#include <type_traits>
 
 #include "hdcm_common.h"
 
@@ -123,19 +126,34 @@ __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_
     }
     return q;
   };
-  // g0..g3 = go[t .. t+3], x0..x2 = x[t .. t+2]; gn = go[t+4] and xn = x[t+3] are in flight or landed, ga
-  // and xa the rows after them; r0 = res[t]
-  uint4 g0[NG], g1[NG], g2[NG], g3[NG], gn[NG], x0[NG], x1[NG], x2[NG], xn[NG], r0[NG];
-  fetch(x0, xb, x_rs, t0);
-  fetch(x1, xb, x_rs, t0 + 1);
-  fetch(g0, gb, g_rs, t0);
-  fetch(g1, gb, g_rs, t0 + 1);
-  fetch(g2, gb, g_rs, t0 + 2);
-  fetch(g3, gb, g_rs, t0 + 3);
-  fetch(x2, xb, x_rs, t0 + 2);
-  fetch(gn, gb, g_rs, t0 + 4);
-  fetch(xn, xb, x_rs, t0 + 3);
-  if (rb) fetch(r0, rb, r_rs, t0);
+  // Rings over rows, indexed by the row's number in the run modulo 4 (2 for gr), so that no step moves
+  // registers: gf = go[t .. t+3] unpacked, gr = go[t+4], go[t+5] and x = x[t .. t+3] as loaded, the last in
+  // flight; r = res[t], res[t+1]
+  float gf[4][NG][E];
+  uint4 gr[2][NG], xr[4][NG], r[2][NG];
+  // go[t] unpacked; columns past the row and rows past the sequence are zeros
+  auto unpack_go = [&](float (&f)[NG][E], const uint4 (&raw)[NG], int t) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      const bool ok = own[i] && t < L;
+      const uint4 v = raw[i];
+      unpack16<T>(ok ? v : make_uint4(0, 0, 0, 0), f[i]);
+    }
+  };
+  fetch(xr[0], xb, x_rs, t0);
+  fetch(xr[1], xb, x_rs, t0 + 1);
+  {
+    uint4 g[4][NG];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) fetch(g[k], gb, g_rs, t0 + k);
+    fetch(xr[2], xb, x_rs, t0 + 2);
+    fetch(gr[0], gb, g_rs, t0 + 4);
+    fetch(xr[3], xb, x_rs, t0 + 3);
+    fetch(gr[1], gb, g_rs, t0 + 5);
+    if (rb) fetch(r[0], rb, r_rs, t0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) unpack_go(gf[k], g[k], t0 + k);
+  }
   float gw[NG][E], cw[4][NG][E];
 #pragma unroll
   for (int i = 0; i < NG; ++i) {
@@ -153,61 +171,41 @@ __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_
   // round for three rows: the gradient sums of t, the variance of t + 1 and the mean of t + 2.
   float mean, mean1, rstd;
   {
-    const float4 m = row_totals(make_float4(sum_of(x0), sum_of(x1), 0.f, 0.f));
+    const float4 m = row_totals(make_float4(sum_of(xr[0]), sum_of(xr[1]), 0.f, 0.f));
     mean = m.x * invD, mean1 = m.y * invD;
-    rstd = rsqrtf(row_totals(make_float4(squares_of(x0, mean), 0.f, 0.f, 0.f)).x * invD + eps);
+    rstd = rsqrtf(row_totals(make_float4(squares_of(xr[0], mean), 0.f, 0.f, 0.f)).x * invD + eps);
   }
   const int t_end = WPR > 1 ? t0 + run_rows : t1;
-#pragma unroll 1
-  for (int t = t0; t < t_end; ++t) {
-    uint4 ga[NG], xa[NG], ra[NG];
-    fetch(ga, gb, g_rs, t + 5);
-    fetch(xa, xb, x_rs, t + 4);
-    if (rb) fetch(ra, rb, r_rs, t + 1);
+  // row t, whose number in the run is M modulo 4
+  auto step = [&](auto M_, int t) {
+    constexpr int M = decltype(M_)::value;
+    if (rb) fetch(r[(M + 1) % 2], rb, r_rs, t + 1);
     const bool in_run = t < t1;
     float xv[NG][E], gh[NG][E];
-#pragma unroll
-    for (int i = 0; i < NG; ++i) {
-      unpack16<T>(x0[i], xv[i]);
-#pragma unroll
-      for (int e = 0; e < E; ++e) xv[i][e] = own[i] ? xv[i][e] - mean : 0.f;
-    }
-    const float rx = in_run ? rstd : 0.f;
+    const float rx = in_run ? rstd : 0.f, in = in_run ? 1.f : 0.f;
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
-      // a lane past the row takes xh = 0, but its taps and go are a neighbour's: go is zeroed
-      const bool ok0 = own[i] && in_run;
-      const uint4 zero = make_uint4(0, 0, 0, 0);
-      float ge[E];
-      unpack16<T>(ok0 ? g0[i] : zero, ge);
+      unpack16<T>(xr[M][i], xv[i]);
+#pragma unroll
+      for (int e = 0; e < E; ++e) xv[i][e] = own[i] ? (xv[i][e] - mean) * rx : 0.f;  // xh
+    }
+    fetch(xr[M], xb, x_rs, t + 4);
+#pragma unroll
+    for (int i = 0; i < NG; ++i)
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        xv[i][e] *= rx;  // xh
-        gh[i][e] = cw[3][i][e] * ge[e];
-        X[3][i][e] += xv[i][e] * ge[e];
-        Gs[i][e] += ge[e];
-      }
-      auto tap = [&](const uint4& g, int k) {
-        float gk[E];
-        unpack16<T>(own[i] && t + k < L ? g : zero, gk);
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          gh[i][e] += cw[3 - k][i][e] * gk[e];
-          X[3 - k][i][e] += xv[i][e] * gk[e];
-        }
-      };
-      tap(g1[i], 1);
-      tap(g2[i], 2);
-      tap(g3[i], 3);
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        gh[i][e] *= gw[i][e];
+        const float f0 = gf[M][i][e], f1 = gf[(M + 1) % 4][i][e], f2 = gf[(M + 2) % 4][i][e], f3 = gf[(M + 3) % 4][i][e];
+        X[3][i][e] += xv[i][e] * f0;
+        X[2][i][e] += xv[i][e] * f1;
+        X[1][i][e] += xv[i][e] * f2;
+        X[0][i][e] += xv[i][e] * f3;
+        Gs[i][e] += in * f0;
+        gh[i][e] = (cw[3][i][e] * f0 + cw[2][i][e] * f1 + cw[1][i][e] * f2 + cw[0][i][e] * f3) * gw[i][e];
         s1 += gh[i][e];
         s2 += gh[i][e] * xv[i][e];
       }
-    }
-    const float4 tot = row_totals(make_float4(s1, s2, squares_of(x1, mean1), sum_of(x2)));
+    const float4 tot = row_totals(make_float4(s1, s2, squares_of(xr[(M + 1) % 4], mean1), sum_of(xr[(M + 2) % 4])));
     const float m1 = tot.x * invD, m2 = tot.y * invD;
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
@@ -216,17 +214,23 @@ __global__ __launch_bounds__(kWpb* kWave, NG * Vec<T>::N > 8 ? 1 : 2) void norm_
       for (int e = 0; e < E; ++e) o[e] = rstd * (gh[i][e] - m1 - xv[i][e] * m2);
       if (rb) {
         float rv[E];
-        unpack16<T>(r0[i], rv);
+        unpack16<T>(r[M % 2][i], rv);
 #pragma unroll
         for (int e = 0; e < E; ++e) o[e] += rv[e];
-        r0[i] = ra[i];
       }
       if (own[i] && in_run) store16<T>(db + (int64_t)t * d_rs + (int64_t)(lane + CW * i) * E, o);
-      g0[i] = g1[i], g1[i] = g2[i], g2[i] = g3[i], g3[i] = gn[i], gn[i] = ga[i];
-      x0[i] = x1[i], x1[i] = x2[i], x2[i] = xn[i], xn[i] = xa[i];
     }
+    unpack_go(gf[M], gr[M % 2], t + 4);
+    fetch(gr[M % 2], gb, g_rs, t + 6);
     mean = mean1, mean1 = tot.w * invD;
     rstd = rsqrtf(tot.z * invD + eps);
+  };
+#pragma unroll 1
+  for (int t = t0; t < t_end; t += 4) {
+    step(std::integral_constant<int, 0>{}, t);
+    if (t + 1 < t_end) step(std::integral_constant<int, 1>{}, t + 1);
+    if (t + 2 < t_end) step(std::integral_constant<int, 2>{}, t + 2);
+    if (t + 3 < t_end) step(std::integral_constant<int, 3>{}, t + 3);
   }
 
   // this workgroup's sums: part[block][5][D] (X_0 .. X_3, G)

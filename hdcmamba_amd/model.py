@@ -169,10 +169,13 @@ class BlockTrainFunction(torch.autograd.Function):
     def forward(ctx, block, x, pad, *params):
         ctx.block, ctx.x, ctx.pad, ctx.mixer = block, x, pad, block.differentiable_mixer
         ctx.autocast = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+        if any(ctx.needs_input_grad[3:]):  # freed after a backward without retain_graph, so a second one raises
+            ctx.save_for_backward(x.new_empty(0))
         return block._native_padded(x, pad)
 
     @staticmethod
     def backward(ctx, dy):
+        _ = ctx.saved_tensors
         block, x, pad = ctx.block, ctx.x, ctx.pad
         need = ctx.needs_input_grad
         params = block._grad_params(ctx.mixer)

@@ -396,6 +396,26 @@ def test_native_training_is_the_composition(dev, dtype, L, mixer):
         assert not blk(x)[0].requires_grad
 
 
+@pytest.mark.parametrize("mixer", [True, False])
+def test_native_training_second_backward(dev, mixer):
+    """A second backward through a freed graph raises, as through the checkpointed composition;
+    with retain_graph it gives the same gradients again."""
+    from hdcmamba_amd import HdcMamba9v3Block
+
+    _say("native training, second backward", mixer)
+    torch.manual_seed(0)
+    blk = HdcMamba9v3Block(256, 64, 4, 64, differentiable_mixer=mixer).to(dev).train()
+    x = torch.randn(1, 70, 256, device=dev, requires_grad=True)
+    for _ in range(2):  # the native path, then the composition
+        y = blk(x)[0].sum()
+        a = torch.autograd.grad(y, [x, blk.out_proj.weight], retain_graph=True)
+        b = torch.autograd.grad(y, [x, blk.out_proj.weight])
+        assert all(max_rel(s, t) <= 1e-5 for s, t in zip(a, b))
+        with pytest.raises(RuntimeError, match="second time"):
+            torch.autograd.grad(y, [x, blk.out_proj.weight])
+        _composition(blk)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_pad_rows_and_gamma(dev, dtype):
     """The padding kernel against F.pad (a batch-strided view, no rows of padding, a width of one

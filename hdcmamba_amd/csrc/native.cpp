@@ -445,10 +445,11 @@ std::vector<Tensor> norm_conv_backward(const Tensor& go_, const Tensor& x_, cons
   return {g.first, w.narrow(0, 0, D), w.narrow(0, D, D), w.narrow(0, 2 * D, 4 * D).view(cw.sizes()), w.narrow(0, 6 * D, D)};
 }
 
-// Weight gradient y^T x of row-major y [M, N], x [M, K] and, with sums, y's column sums
-std::pair<Tensor, Tensor> weight_grad(const Tensor& y, const Tensor& x, bool sums, bool library, void* s) {
+// Weight gradient y^T x of row-major y [M, N], x [M, K] and, with sums, y's column sums.  By the rule on sizes
+// also where recorded library solutions are in use: those are of the forward's products.
+std::pair<Tensor, Tensor> weight_grad(const Tensor& y, const Tensor& x, bool sums, void* s) {
   const int64_t M = y.size(0), N = y.size(1), K = x.size(1);
-  if (library || !hdcm_gemm_tn_preferred(M, N, K, sums, dtype_of(y)) || !aligned(y, 16) || !aligned(x, 16))
+  if (!hdcm_gemm_tn_preferred(M, N, K, sums, dtype_of(y)) || !aligned(y, 16) || !aligned(x, 16))
     return {at::mm(y.t(), x), sums ? y.sum(0) : Tensor()};
   Tensor w = at::empty({N, K}, y.options()), c = sums ? at::empty({N}, y.options()) : Tensor();
   const size_t n = hdcm_gemm_tn_workspace_bytes(M, N, K);
@@ -489,7 +490,7 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
   if (need[11]) {
     Tensor c = at::empty_like(m.combined);
     row_norm(m.combined, c, st.main);
-    give(10, weight_grad(dy2, c.view({M, K}), false, library, st.main).first);
+    give(10, weight_grad(dy2, c.view({M, K}), false, st.main).first);
   }
   if (!mixer_grad) {
     if (need[0]) out[0] = dy;
@@ -514,7 +515,7 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
   }
   const Tensor dproj2 = g.first.view({M, N});
   if (need[5]) {
-    const auto wg = weight_grad(dproj2, m.x_conv.view({M, dm}), need[6], library, st.main);
+    const auto wg = weight_grad(dproj2, m.x_conv.view({M, dm}), need[6], st.main);
     give(4, wg.first);
     if (need[6]) give(5, wg.second);
   } else if (need[6]) {

@@ -287,13 +287,13 @@ __global__ __launch_bounds__(kSumC* kSumR) void norm_conv_bwd_sum_kernel(
 #pragma unroll
   for (int m = 0; m < 5; ++m) acc[j][m][x] = s[m];
   __syncthreads();
-  if (j < 5) {  // slice sums of value j, in order
+  // Slice sums of value j, in order.  A thread reads and overwrites its own column acc[.][j][x] only, so
+  // nothing is waited for in between (and j = 4 and j = 5 share a wave: a barrier in here would be
+  // passed twice by it).
+  if (j < 5) {
     float t = 0.f;
     for (int r = 0; r < kSumR; ++r) t += acc[r][j][x];
-    __syncthreads();
     acc[0][j][x] = t;
-  } else {
-    __syncthreads();
   }
   __syncthreads();
   if (j == 0 && c < D) {

@@ -88,6 +88,22 @@ def test_norm_conv_backward_runs(dev, dtype, B, L, D):
         assert max_rel(a, e) <= 1e-4, (name, max_rel(a, e))
 
 
+@pytest.mark.parametrize("dtype,B,L,D", [(torch.bfloat16, 1, 9001, 520), (torch.float32, 3, 700, 260)])
+def test_norm_conv_backward_sums_exact(dev, dtype, B, L, D):
+    """The sums over the workgroups' rows with whole numbers as grad_out: their column sums are below
+    2^24, so d_conv_b is exact whatever the order (more workgroups than the 64 slices that add them,
+    a last block of 16 columns that is not full)."""
+    _say("norm_conv bwd exact sums", dtype, B, L, D)
+    g = torch.Generator(device=dev).manual_seed(D)
+    x = torch.randn(B, L, D, generator=g, device=dev).to(dtype)
+    go = torch.randint(-8, 9, (B, L, D), generator=g, device=dev).to(dtype)
+    w, cw = torch.ones(D, device=dev, dtype=dtype), torch.ones(D, 1, 4, device=dev, dtype=dtype)
+    _, _, d_ln_b, _, d_conv_b = _ops.norm_conv_bwd(go, x, w, w, cw, 1e-5)
+    ref = go.double().sum((0, 1))
+    assert torch.equal(d_conv_b.double(), ref)
+    assert torch.equal(d_ln_b.double(), 4 * ref)
+
+
 @pytest.mark.parametrize("dtype,B,L,D", [(torch.bfloat16, 2, 1, 256), (torch.bfloat16, 3, 37, 1024), (torch.bfloat16, 1, 130, 2048),
                                          (torch.float32, 2, 2, 128), (torch.float32, 1, 67, 768), (torch.float32, 1, 35, 3072)])
 def test_norm_conv_backward_add(dev, dtype, B, L, D):

@@ -171,7 +171,7 @@ class BlockTrainFunction(torch.autograd.Function):
         ctx.autocast = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
         if any(ctx.needs_input_grad[3:]):  # freed after a backward without retain_graph, so a second one raises
             ctx.save_for_backward(x.new_empty(0))
-        return block._native_padded(x, pad)
+        return block._native_padded(x, pad, train=True)
 
     @staticmethod
     def backward(ctx, dy):
@@ -390,22 +390,25 @@ class HdcMamba9v3Block(nn.Module):
     def _native_streams(self, x):
         return _ops.native_streams(x, x.shape[1], self.d_state, self.ssm_overlap)
 
-    def _native_forward(self, x, state=None, out=None):
-        """The block body on chunk-aligned contiguous x without autograd (_inner_forward)."""
+    def _native_forward(self, x, state=None, out=None, train=False):
+        """The block body on chunk-aligned contiguous x without autograd (_inner_forward).  ``train``: as
+        the composition runs with autograd, the row LayerNorm in a pass of its own before out_proj
+        (two-pass variance, the weight as it is now: the folded form reads row sums kept until the
+        weight's version changes, which a write through ``.data`` or a flat buffer does not do)."""
         w = self.out_proj.weight
-        fused = self._fused_out(x)
+        fused = not train and self._fused_out(x)
         sums = self._out_weight_sums(w.to(x.dtype)) if fused and _ops.rowln_stats_ok(x, self.d_model) else None
         return _ops.native().block_forward(
             x, self._params(), self.norm.eps, (self.d_state, self.num_heads, self.chunk_size), self._native_streams(x),
             out, fused, sums, torch.cuda.tunable.is_enabled(), None if state is None else state.h,
             None if state is None else state.S_prev)
 
-    def _native_padded(self, x, pad):
+    def _native_padded(self, x, pad, train=False):
         """_native_forward on x [B,L,dm] with ``pad`` zero rows in front, which the output leaves out."""
         if not pad:
-            return self._native_forward(x.contiguous())
+            return self._native_forward(x.contiguous(), train=train)
         xp = _ops.native().pad_rows(x, pad, _ops._stream(x))
-        return self._native_forward(xp, out=xp)[:, pad:, :]
+        return self._native_forward(xp, out=xp, train=train)[:, pad:, :]
 
     def _fused_out(self, x):
         """Whether out_proj runs as the GEMM with the LayerNorm folded in (bf16, no autograd).
@@ -620,7 +623,7 @@ class HdcMamba9v3Block(nn.Module):
                 if x.requires_grad or any(p.requires_grad for p in params):
                     return BlockTrainFunction.apply(self, x, pad, *params), None
                 with torch.no_grad():
-                    return self._native_padded(x, pad), None
+                    return self._native_padded(x, pad, train=True), None
         if pad > 0:
             x = F.pad(x, (0, 0, pad, 0))
         if self.training:

@@ -1,0 +1,83 @@
+"""What the native host path owes its callers beyond equal values: every test runs on it and on the
+Python composition of the same kernels, which states what is right, refused or accepted."""
+import weakref
+
+import pytest
+import torch
+
+from cfgs import max_rel, reinit_block_
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(*a):
+    print(*a, flush=True)
+
+
+def _block(dev, dtype=torch.float32, mixer=False, dm=256, ds=64, H=4, C=64, seed=3):
+    from hdcmamba_amd import HdcMamba9v3Block
+
+    torch.manual_seed(0)
+    blk = reinit_block_(HdcMamba9v3Block(dm, ds, H, C, differentiable_mixer=mixer), seed=seed, decays_uniform=True)
+    return blk.to(dtype).to(dev).train()
+
+
+def _x(dev, L, dtype=torch.float32, B=2, dm=256, seed=5):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return torch.randn(B, L, dm, generator=g, device=dev).to(dtype)
+
+
+def _paths(blk):
+    """blk on the native host path, then on the composition."""
+    yield "native"
+    blk._native_ok = lambda x: False
+    yield "composition"
+    del blk._native_ok
+
+
+LIM = {torch.float32: 1e-5, torch.bfloat16: 1.5e-2}  # as test_native_training_is_the_composition
+
+
+@pytest.mark.parametrize("mixer", [False, True])
+@pytest.mark.parametrize("how", ["data", "pointer"])
+def test_training_reads_the_weight_of_the_call(dev, mixer, how):
+    """A training forward uses out_proj's weight as it is at the call, whatever changed it: a write
+    through ``.data`` or into the storage leaves the version counter alone.  The rows of `combined`
+    have a mean of about 1 (GroupNorm's bias) and the weight's rows a sum, so stale row sums would
+    show."""
+    _say("training weight", mixer, how)
+    blk = _block(dev, torch.bfloat16, mixer)
+    with torch.no_grad():
+        blk.group_norm.bias.add_(2.0)
+        blk.in_proj.bias[3 * 64 + 3 * 256:] += 3.0
+        blk.out_proj.weight.add_(0.02)
+    w0 = blk.out_proj.weight.detach().clone()
+    x = _x(dev, 100, torch.bfloat16)
+    out = {}
+    for path in _paths(blk):
+        with torch.no_grad():
+            blk.out_proj.weight.copy_(w0)
+        blk(x)
+        w = blk.out_proj.weight
+        if how == "data":
+            w.data.mul_(-1.5)
+        else:
+            torch.empty(0, dtype=w.dtype, device=dev).set_(w.untyped_storage(), 0, w.shape).mul_(-1.5)
+        out[path] = blk(x)[0].detach()
+    assert max_rel(out["native"], out["composition"]) <= LIM[torch.bfloat16]
+
+
+def test_training_out_proj_is_the_composition(dev):
+    """The training forward normalises `combined` in a pass of its own (two-pass variance) before
+    out_proj, also where nothing requires a gradient: bit-identical to the composition."""
+    _say("training out_proj")
+    blk = _block(dev, torch.bfloat16)
+    x = _x(dev, 128, torch.bfloat16)
+    out = {}
+    for path in _paths(blk):
+        blk.requires_grad_(True)
+        a = blk(x)[0].detach()
+        blk.requires_grad_(False)
+        out[path] = a, blk(x)[0]
+    assert torch.equal(out["native"][0], out["composition"][0])
+    assert torch.equal(out["native"][1], out["composition"][1])

@@ -171,7 +171,8 @@ class BlockTrainFunction(torch.autograd.Function):
         ctx.autocast = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
         if any(ctx.needs_input_grad[3:]):  # freed after a backward without retain_graph, so a second one raises
             ctx.save_for_backward(x.new_empty(0))
-        return block._native_padded(x, pad, train=True)
+        # .data: a tensor of its own on that storage.  A view made in here could not be changed in place.
+        return block._native_padded(x, pad, train=True).data
 
     @staticmethod
     def backward(ctx, dy):

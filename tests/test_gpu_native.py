@@ -81,3 +81,18 @@ def test_training_out_proj_is_the_composition(dev):
         out[path] = a, blk(x)[0]
     assert torch.equal(out["native"][0], out["composition"][0])
     assert torch.equal(out["native"][1], out["composition"][1])
+
+
+@pytest.mark.parametrize("L", [128, 100])
+def test_training_output_changed_in_place(dev, L):
+    """The training output may be changed in place (a residual added to it), padded or not."""
+    _say("training output in place", L)
+    blk = _block(dev, mixer=True)
+    grads = []
+    for path in _paths(blk):
+        x = _x(dev, L).requires_grad_()
+        y, _ = blk(x)
+        y += x
+        y *= 2.0
+        grads.append(torch.autograd.grad(y, [x, blk.out_proj.weight, blk.in_proj.weight], torch.ones_like(y)))
+    assert all(max_rel(a, b) <= 1e-5 for a, b in zip(*grads))

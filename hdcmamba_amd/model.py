@@ -155,55 +155,70 @@ class SlotSsmMixerFunction(torch.autograd.Function):
         return dprojs, dA, None, dgw, dgb, None, None, None, None
 
 
+class _PadRows(torch.autograd.Function):
+    """x [B,L,dm] with ``pad`` zero rows in front of every sequence (hdcm_pad_rows_fwd)."""
+
+    @staticmethod
+    def forward(ctx, x, pad):
+        ctx.pad = pad
+        return _ops.native().pad_rows(x, pad, _ops._stream(x))
+
+    @staticmethod
+    def backward(ctx, g):
+        return g[:, ctx.pad:, :], None
+
+
 class BlockTrainFunction(torch.autograd.Function):
     """One block's training forward and its backward as two native calls: the forward keeps the
     block and its input only and the backward recomputes the body from the block's parameters of
     that moment, as the reference's checkpoint does (model.py:391-392).
 
-    ``apply(block, x, pad, *params)`` on the unpadded x [B,L,dm], params those of
-    ``block._grad_params()``.  A backward that is itself to be differentiated
-    (create_graph) runs through the block's Python composition instead.
+    ``apply(block, x, pad, *params)`` on the chunk-aligned contiguous x [B, pad + L, dm] of which the
+    output leaves out the first ``pad`` rows; params those of ``block._grad_params()``.  x is saved
+    only where the backward needs the body (not where only x gets a gradient, which is dy, and the
+    mixer is not differentiated).  A backward that is itself to be differentiated (create_graph)
+    runs through the block's Python composition instead.
     """
 
     @staticmethod
     def forward(ctx, block, x, pad, *params):
-        ctx.block, ctx.x, ctx.pad, ctx.mixer = block, x, pad, block.differentiable_mixer
+        ctx.block, ctx.pad, ctx.mixer = block, pad, block.differentiable_mixer
         ctx.autocast = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
-        if any(ctx.needs_input_grad[3:]):  # freed after a backward without retain_graph, so a second one raises
-            ctx.save_for_backward(x.new_empty(0))
+        ctx.body = ctx.mixer or ctx.needs_input_grad[3]
+        ctx.dtype = x.dtype
+        if ctx.body:
+            ctx.save_for_backward(x)
+        y = block._native_forward(x, train=True)
         # .data: a tensor of its own on that storage.  A view made in here could not be changed in place.
-        return block._native_padded(x, pad, train=True).data
+        return y[:, pad:, :].data if pad else y
 
     @staticmethod
     def backward(ctx, dy):
-        _ = ctx.saved_tensors
-        block, x, pad = ctx.block, ctx.x, ctx.pad
+        block, pad = ctx.block, ctx.pad
         need = ctx.needs_input_grad
+        if not ctx.body:
+            return None, F.pad(dy.to(ctx.dtype), (0, 0, pad, 0)), None, None
+        (x,) = ctx.saved_tensors
         params = block._grad_params(ctx.mixer)
         if torch.is_grad_enabled():
             with torch.enable_grad(), torch.amp.autocast("cuda", dtype=ctx.autocast[1], enabled=ctx.autocast[0]):
-                y = block._inner_forward(F.pad(x, (0, 0, pad, 0)).contiguous())[:, pad:, :]
+                y = block._inner_forward(x)[:, pad:, :]
             wanted = [t for t, n in zip((x, *params), (need[1], *need[3:])) if n]
             grads = iter(torch.autograd.grad(y, wanted, dy, create_graph=True, allow_unused=True))
             dx = next(grads) if need[1] else None
             return (None, dx, None, *(next(grads) if n else None for n in need[3:]))
         native = _ops.native()
-        dt, stream = x.dtype, _ops._stream(x)
-        dyp = dy.to(dt)
-        if pad:
-            x, dyp = native.pad_rows(x, pad, stream), native.pad_rows(dyp, pad, stream)
-        else:
-            x, dyp = x.contiguous(), dyp.contiguous()
+        dyp = dy.to(ctx.dtype)
+        dyp = native.pad_rows(dyp, pad, _ops._stream(x)) if pad else dyp.contiguous()
         if ctx.mixer:
             mask = [need[1], *need[3:10], False, *need[10:]]
         else:
             mask = [need[1], *[False] * 10, need[3]]
         g = native.block_backward(x, dyp, block._params(), block.norm.eps, (block.d_state, block.num_heads, block.chunk_size),
                                   block._native_streams(x), ctx.mixer, torch.cuda.tunable.is_enabled(), mask)
-        dx = g[0][:, pad:, :] if g[0] is not None and pad else g[0]
         if ctx.mixer:
-            return (None, dx, None, *g[1:8], *g[9:])
-        return None, dx, None, g[11]
+            return (None, g[0], None, *g[1:8], *g[9:])
+        return None, g[0], None, g[11]
 
 
 class HdcMamba9v3Block(nn.Module):
@@ -622,7 +637,8 @@ class HdcMamba9v3Block(nn.Module):
             if self.training:
                 params = self._grad_params()
                 if x.requires_grad or any(p.requires_grad for p in params):
-                    return BlockTrainFunction.apply(self, x, pad, *params), None
+                    xp = _PadRows.apply(x, pad) if pad else x.contiguous()
+                    return BlockTrainFunction.apply(self, xp, pad, *params), None
                 with torch.no_grad():
                     return self._native_padded(x, pad, train=True), None
         if pad > 0:

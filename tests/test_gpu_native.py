@@ -83,6 +83,83 @@ def test_training_out_proj_is_the_composition(dev):
     assert torch.equal(out["native"][1], out["composition"][1])
 
 
+@pytest.mark.parametrize("mixer", [False, True])
+def test_training_input_changed_in_place(dev, mixer):
+    """x changed between forward and backward: refused where the forward kept x itself, and without
+    effect where it kept a copy of its own (padded or not contiguous)."""
+    _say("training input in place", mixer)
+    blk = _block(dev, mixer=mixer)
+    grads = {}
+    for path in _paths(blk):
+        x = _x(dev, 128)
+        y = blk(x)[0].sum()
+        x.add_(1.0)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.backward()
+        for L, view in ((100, lambda t: t), (128, lambda t: t.transpose(0, 1).contiguous().transpose(0, 1))):
+            for change in (False, True):
+                x = view(_x(dev, L))
+                y = blk(x)[0].square().sum()
+                if change:
+                    x.add_(1.0)
+                (grads[path, L, change],) = torch.autograd.grad(y, [blk.out_proj.weight])
+    for (path, L, _), g in grads.items():
+        assert max_rel(g, grads["composition", L, False]) <= 1e-4, (path, L)
+
+
+@pytest.mark.parametrize("mixer,L", [(False, 128), (True, 128), (True, 100)])
+def test_training_input_is_freed_and_hooked(dev, mixer, L):
+    """The kept input goes through saved-tensor hooks, and is given back when the backward has run,
+    not with the graph."""
+    _say("training input kept", mixer, L)
+    blk = _block(dev, mixer=mixer)
+    for path in _paths(blk):
+        seen = []
+
+        def pack(t):
+            seen.append(tuple(t.shape))
+            return t.cpu()
+
+        leaf = _x(dev, L).requires_grad_()
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(dev)):
+            h = leaf * 1.0
+            y = blk(h)[0].sum()
+        assert (2, 128, 256) in seen, path
+        a = torch.autograd.grad(y, [leaf, blk.out_proj.weight])
+        h = leaf * 1.0
+        y = blk(h)[0].sum()
+        alive = weakref.ref(h)
+        del h
+        b = torch.autograd.grad(y, [leaf, blk.out_proj.weight])
+        assert alive() is None, path
+        assert all(max_rel(s, t) <= 1e-5 for s, t in zip(a, b)), path
+
+
+@pytest.mark.parametrize("mixer,L", [(False, 128), (False, 100), (True, 128), (True, 100)])
+def test_training_backward_with_frozen_parameters(dev, mixer, L):
+    """With x alone requiring a gradient: the differentiable mixer keeps x, so a second backward through
+    the freed graph raises; without it the gradient is dy itself, nothing is kept, and a second
+    backward and a changed x are accepted."""
+    _say("frozen parameters", mixer, L)
+    blk = _block(dev, mixer=mixer).requires_grad_(False)
+    grads = []
+    for path in _paths(blk):
+        x = _x(dev, L).requires_grad_()
+        h = x + 0.0  # (keeps nothing itself)
+        y = blk(h)[0].square().sum()
+        grads.append(torch.autograd.grad(y, [x], retain_graph=True)[0])
+        if mixer:
+            torch.autograd.grad(y, [x])
+            with pytest.raises(RuntimeError, match="second time"):
+                torch.autograd.grad(y, [x])
+        else:
+            z = blk(h)[0].sum()
+            h.add_(1.0)
+            for _ in range(2):
+                assert torch.equal(torch.autograd.grad(z, [x])[0], torch.ones_like(x)), path
+    assert max_rel(*grads) <= 1e-5
+
+
 @pytest.mark.parametrize("L", [128, 100])
 def test_training_output_changed_in_place(dev, L):
     """The training output may be changed in place (a residual added to it), padded or not."""
@@ -96,3 +173,19 @@ def test_training_output_changed_in_place(dev, L):
         y *= 2.0
         grads.append(torch.autograd.grad(y, [x, blk.out_proj.weight, blk.in_proj.weight], torch.ones_like(y)))
     assert all(max_rel(a, b) <= 1e-5 for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("L", [128, 100])
+def test_training_second_derivative(dev, L):
+    """A gradient of a gradient with respect to x goes on to what x was made from, padded or not."""
+    _say("second derivative", L)
+    blk = _block(dev)
+    res = []
+    for path in _paths(blk):
+        s = torch.ones((), device=dev, requires_grad=True)
+        x = _x(dev, L)
+        y, _ = blk(x * s)
+        (gs,) = torch.autograd.grad((y ** 3).sum(), [s], create_graph=True)
+        res.append(torch.stack([gs.detach(), torch.autograd.grad(gs, [s])[0]]))
+    assert torch.isfinite(res[0]).all()
+    assert ((res[0] - res[1]).abs() <= 1e-4 * res[1].abs()).all()

@@ -34,6 +34,13 @@ int dtype_of(const Tensor& t) {
   return HDCM_F32;
 }
 
+// Held by every entry point: no autograd, and no autocast, which would give a product another dtype than
+// the kernels around it are told (a backward may be called inside a region that its forward was not in).
+struct Entry {
+  at::NoGradGuard no_grad;
+  c10::impl::ExcludeDispatchKeyGuard no_autocast{c10::autocast_dispatch_keyset};
+};
+
 void on_gpu(const Tensor& t) {
   TORCH_CHECK(t.is_cuda(), "hdcmamba_amd kernels need ROCm GPU tensors; got a tensor on ", t.device(),
               " (there is no CPU path)");
@@ -258,7 +265,7 @@ float* opt_ptr(const OptTensor& t, at::IntArrayRef shape, const char* name) {
 Tensor block_forward(const Tensor& x, const std::vector<Tensor>& params, double eps, const DimArgs& dims,
                      const StreamArgs& streams, const OptTensor& out, bool fused, const OptTensor& w_sums, bool library,
                      const OptTensor& h_final, const OptTensor& S_final) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(x);
   const Dims d = dims_of(dims);
   const int64_t B = x.size(0), dm = x.size(2), hd = dm / d.H;
@@ -269,7 +276,7 @@ Tensor block_forward(const Tensor& x, const std::vector<Tensor>& params, double 
 
 // [B, pad + L, dm] with pad zero rows in front of every sequence's rows
 Tensor pad_rows(const Tensor& x_, int64_t pad, int64_t stream) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(x_);
   const int dt = dtype_of(x_);
   const int64_t E = dt == HDCM_BF16 ? 8 : 4;
@@ -299,7 +306,7 @@ void refresh_gamma(const Tensor& decay_log, const Tensor& gamma, int64_t stream)
 Tensor block_step(const Tensor& x_, const std::vector<Tensor>& params, double eps, const DimArgs& dims, const Tensor& conv,
                   const Tensor& h, const Tensor& S_prev, const Tensor& S_intra, int64_t pos, const OptTensor& pos_dev,
                   bool fused_front, bool fused_out, const OptTensor& step_ws, int64_t stream) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(x_);
   const Dims d = dims_of(dims);
   Tensor x = x_.stride(1) == 1 && x_.stride(0) % 8 == 0 && (uintptr_t)x_.const_data_ptr() % 16 == 0 ? x_ : x_.contiguous();
@@ -392,7 +399,7 @@ std::pair<Tensor, Tensor> mixer_grads(const Tensor& projs, const Tensor& A_log, 
 // SlotSsmMixerFunction: (combined, slot workspace) from projs [B, L, P]
 std::vector<Tensor> mixer_forward(const Tensor& projs, const Tensor& A_log, const Tensor& gamma, const Tensor& gnw,
                                   const Tensor& gnb, const DimArgs& dims, const StreamArgs& streams) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(projs);
   Params p;
   p.A_log = same(A_log, projs, "A_log");
@@ -409,7 +416,7 @@ std::vector<Tensor> mixer_forward(const Tensor& projs, const Tensor& A_log, cons
 std::vector<Tensor> mixer_backward(const Tensor& dcomb_, const Tensor& projs, const Tensor& A_log, const Tensor& gamma,
                                    const Tensor& gnw, const Tensor& gnb, const Tensor& combined, const Tensor& slot_ws,
                                    const DimArgs& dims, int64_t stream) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(dcomb_);
   const Tensor dcomb = same(dcomb_, projs, "grad");
   const Dims d = dims_of(dims);
@@ -424,7 +431,7 @@ std::vector<Tensor> mixer_backward(const Tensor& dcomb_, const Tensor& projs, co
 // FusedNormConv1dFunction
 Tensor norm_conv_forward(const Tensor& x_, const Tensor& nw, const Tensor& nb, const Tensor& cw, const Tensor& cb,
                          double eps, int64_t stream) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(x_);
   TORCH_CHECK(x_.dim() == 3, "norm_conv expects x of shape [B, L, D]");
   const Tensor x = x_.stride(2) == 1 ? x_ : x_.contiguous();
@@ -435,7 +442,7 @@ Tensor norm_conv_forward(const Tensor& x_, const Tensor& nw, const Tensor& nb, c
 
 std::vector<Tensor> norm_conv_backward(const Tensor& go_, const Tensor& x_, const Tensor& nw, const Tensor& nb,
                                        const Tensor& cw, double eps, int64_t stream) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(go_);
   const Tensor x = x_.stride(2) == 1 ? x_ : x_.contiguous();
   const int64_t D = x.size(2);
@@ -468,7 +475,7 @@ std::pair<Tensor, Tensor> weight_grad(const Tensor& y, const Tensor& x, bool sum
 std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const std::vector<Tensor>& params, double eps,
                                       const DimArgs& dims, const StreamArgs& streams, bool mixer_grad, bool library,
                                       const std::vector<bool>& need) {
-  at::NoGradGuard no_grad;
+  Entry entry;
   on_gpu(x);
   const Dims d = dims_of(dims);
   const Streams st = streams_of(streams);

@@ -189,3 +189,20 @@ def test_training_second_derivative(dev, L):
         res.append(torch.stack([gs.detach(), torch.autograd.grad(gs, [s])[0]]))
     assert torch.isfinite(res[0]).all()
     assert ((res[0] - res[1]).abs() <= 1e-4 * res[1].abs()).all()
+
+
+@pytest.mark.parametrize("mixer", [False, True])
+@pytest.mark.parametrize("dtype,region", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float16)])
+def test_training_backward_in_an_autocast_region(dev, mixer, dtype, region):
+    """A backward called inside an autocast region that the forward was not in computes in the
+    forward's types: the same gradients as outside."""
+    _say("backward under autocast", mixer, dtype, region)
+    blk = _block(dev, dtype, mixer)
+    x = _x(dev, 100, dtype).requires_grad_()
+    dy = _x(dev, 100, dtype, seed=6)
+    params = [x, blk.out_proj.weight] + ([blk.in_proj.weight, blk.norm.weight, blk.A_log] if mixer else [])
+    want = torch.autograd.grad(blk(x)[0], params, dy)
+    y = blk(x)[0]
+    with torch.amp.autocast("cuda", dtype=region):
+        got = torch.autograd.grad(y, params, dy)
+    assert all(a.dtype == b.dtype and torch.equal(a, b) for a, b in zip(got, want))

@@ -845,7 +845,7 @@ def mixer_step(projs, A_log, d_state, q_col, gamma, gn_w, gn_b, gn_eps, h, S_pre
     projs [B,P]; h [B,ds], S_prev / S_intra [B,H,hd,hd] fp32 contiguous, updated in place;
     pos = token offset in its chunk (or, with pos_dev, an int32 device scalar holding it).
     Writes out[:, y_col:y_col+ds] and out[:, g_col:g_col+dm]."""
-    _on_gpu(projs, out, h, S_prev, S_intra)
+    _on_gpu(projs, out, h, S_prev, S_intra, pos_dev)
     B = projs.shape[0]
     if g_col is None:
         g_col = y_col + d_state

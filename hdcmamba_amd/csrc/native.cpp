@@ -255,8 +255,14 @@ ForwardOut forward(const Tensor& x, const Params& p, const Dims& d, const Stream
   return {out, m};
 }
 
-float* opt_ptr(const OptTensor& t, at::IntArrayRef shape, const char* name) {
+void on_device_of(const Tensor& t, const Tensor& ref, const char* name) {
+  TORCH_CHECK(t.device() == ref.device(), name, " is on ", t.device(), ", expected ", ref.device());
+}
+
+// A state the kernels write through its pointer: fp32, contiguous, on x's device.
+float* opt_ptr(const OptTensor& t, at::IntArrayRef shape, const Tensor& x, const char* name) {
   if (!t) return nullptr;
+  on_device_of(*t, x, name);
   TORCH_CHECK(t->scalar_type() == at::kFloat && t->is_contiguous() && t->sizes() == shape, name,
               " must be a contiguous fp32 tensor of shape ", shape);
   return t->mutable_data_ptr<float>();
@@ -270,7 +276,7 @@ Tensor block_forward(const Tensor& x, const std::vector<Tensor>& params, double 
   const Dims d = dims_of(dims);
   const int64_t B = x.size(0), dm = x.size(2), hd = dm / d.H;
   return forward(x, params_of(params, x, eps), d, streams_of(streams), out, fused, w_sums, library,
-                 opt_ptr(h_final, {B, d.ds}, "h"), opt_ptr(S_final, {B, d.H, hd, hd}, "S_prev"))
+                 opt_ptr(h_final, {B, d.ds}, x, "h"), opt_ptr(S_final, {B, d.H, hd, hd}, x, "S_prev"))
       .y;
 }
 
@@ -317,9 +323,11 @@ Tensor block_step(const Tensor& x_, const std::vector<Tensor>& params, double ep
   void* s = (void*)stream;
   TORCH_CHECK(conv.scalar_type() == x.scalar_type() && conv.is_contiguous() && conv.sizes() == at::IntArrayRef({B, 3, dm}),
               "step: conv must be a contiguous [B,3,D] tensor of x's dtype");
-  float* hp = opt_ptr(h, {B, ds}, "h");
-  float* sp = opt_ptr(S_prev, {B, d.H, hd, hd}, "S_prev");
-  float* si = opt_ptr(S_intra, {B, d.H, hd, hd}, "S_intra");
+  on_device_of(conv, x, "conv");
+  if (pos_dev) on_device_of(*pos_dev, x, "pos_dev");
+  float* hp = opt_ptr(h, {B, ds}, x, "h");
+  float* sp = opt_ptr(S_prev, {B, d.H, hd, hd}, x, "S_prev");
+  float* si = opt_ptr(S_intra, {B, d.H, hd, hd}, x, "S_intra");
   Tensor projs = at::empty({B, N}, x.options()), u = at::empty({B, dm}, x.options());
   const bool bf = dt == HDCM_BF16, rows16 = bf && B >= 1 && B <= 16;
   if (fused_front && rows16 && dm % 32 == 0 && dm <= 2048 && N >= 2048) {

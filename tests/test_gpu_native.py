@@ -206,3 +206,22 @@ def test_training_backward_in_an_autocast_region(dev, mixer, dtype, region):
     with torch.amp.autocast("cuda", dtype=region):
         got = torch.autograd.grad(y, params, dy)
     assert all(a.dtype == b.dtype and torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_step_refuses_a_state_elsewhere(dev):
+    """A decode state left on the CPU, wholly or one tensor of it, is an error before any launch."""
+    _say("step state device")
+    blk = _block(dev, torch.bfloat16).eval()
+    x = _x(dev, 64, torch.bfloat16)
+    with torch.no_grad():
+        _, st = blk.prefill(x)
+        for path in _paths(blk):
+            for name in ("conv", "h", "S_prev", "S_intra"):
+                kept = getattr(st, name)
+                setattr(st, name, kept.cpu())
+                with pytest.raises(RuntimeError, match="cpu"):
+                    blk.step(x[:, 0], st)
+                setattr(st, name, kept)
+            assert torch.isfinite(blk.step(x[:, 0], st)).all(), path
+        with pytest.raises(RuntimeError, match="cpu"):
+            blk.step(x[:, 0], st, pos_dev=torch.zeros(1, dtype=torch.int32))

@@ -493,6 +493,20 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
   const auto give = [&](int i, const Tensor& g) {  // i: params_of's index
     if (need[i + 1]) out[i + 1] = g.scalar_type() == params[i].scalar_type() ? g : g.to(params[i].scalar_type());
   };
+  // Parts [start, start + n) of fp32 sums, rounded once, to the type of each parameter (one conversion for
+  // a run of parameters of one type).
+  struct Part {
+    int i;
+    int64_t start, n;
+  };
+  const auto give_sums = [&](const Tensor& sums, std::initializer_list<Part> parts) {
+    Tensor w = sums;
+    for (const Part& q : parts) {
+      if (!need[q.i + 1]) continue;
+      if (w.scalar_type() != params[q.i].scalar_type()) w = sums.to(params[q.i].scalar_type());
+      give(q.i, w.narrow(0, q.start, q.n).view(params[q.i].sizes()));
+    }
+  };
   if (!mixer_grad && !need[11]) {
     if (need[0]) out[0] = dy;
     return out;
@@ -522,12 +536,7 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
   m.projs.reset();
   m.combined.reset();
   dcomb.reset();
-  {
-    const Tensor w = g.second.to(params[8].scalar_type());
-    give(8, w.narrow(0, 0, dm));
-    give(9, w.narrow(0, dm, dm));
-    give(6, w.narrow(0, 2 * dm, d.ds));
-  }
+  give_sums(g.second, {{8, 0, dm}, {9, dm, dm}, {6, 2 * dm, d.ds}});
   const Tensor dproj2 = g.first.view({M, N});
   if (need[5]) {
     const auto wg = weight_grad(dproj2, m.x_conv.view({M, dm}), need[6], st.main);
@@ -541,11 +550,7 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
     const bool add = aligned(dy, 16);
     auto n = norm_conv_bwd(dxc, x, p.nw, p.nb, p.cw, add ? &dy : nullptr, p.eps, st.main);
     if (need[0]) out[0] = add ? n.first : n.first.add_(dy);
-    const Tensor w = n.second.to(params[0].scalar_type());
-    give(0, w.narrow(0, 0, dm));
-    give(1, w.narrow(0, dm, dm));
-    give(2, w.narrow(0, 2 * dm, 4 * dm).view(params[2].sizes()));
-    give(3, w.narrow(0, 6 * dm, dm));
+    give_sums(n.second, {{0, 0, dm}, {1, dm, dm}, {2, 2 * dm, 4 * dm}, {3, 6 * dm, dm}});
   }
   return out;
 }

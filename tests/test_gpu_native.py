@@ -191,6 +191,31 @@ def test_training_second_derivative(dev, L):
     assert ((res[0] - res[1]).abs() <= 1e-4 * res[1].abs()).all()
 
 
+def test_training_gradients_in_the_parameters_types(dev):
+    """Parameters kept in fp32 beside bf16 ones get gradients of fp32 sums that were not rounded to bf16 on
+    the way (A_log and the GroupNorm's among the mixer's)."""
+    _say("mixed parameter types")
+    grads = []
+    blk = _block(dev, torch.bfloat16, mixer=True)
+    blk.A_log.data = blk.A_log.data.float()
+    blk.group_norm.bias.data = blk.group_norm.bias.data.float()
+    x = _x(dev, 128, torch.bfloat16)
+    dy = _x(dev, 128, torch.bfloat16, seed=6)
+    want = [blk.A_log, blk.group_norm.bias, blk.group_norm.weight]
+    g = torch.autograd.grad(blk(x)[0], want, dy)
+    assert [t.dtype for t in g] == [torch.float32, torch.float32, torch.bfloat16]
+    for t in g[:2]:
+        assert not torch.equal(t, t.bfloat16().float())
+    grads.append(g)
+    f = _block(dev, torch.float32, mixer=True)
+    f.load_state_dict(blk.state_dict())
+    f.norm.weight.data = f.norm.weight.data.bfloat16()  # the first of the LayerNorm + conv's
+    h = torch.autograd.grad(f(x.float())[0], [f.norm.weight, f.norm.bias, f.conv1d.weight, f.conv1d.bias], dy.float())
+    assert [t.dtype for t in h] == [torch.bfloat16] + 3 * [torch.float32]
+    for t in h[1:]:
+        assert not torch.equal(t, t.bfloat16().float())
+
+
 @pytest.mark.parametrize("mixer", [False, True])
 @pytest.mark.parametrize("dtype,region", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float16)])
 def test_training_backward_in_an_autocast_region(dev, mixer, dtype, region):

@@ -62,6 +62,11 @@ int64_t row_stride(const Tensor& t, const char* name) {
   return rs;
 }
 
+// Batch stride of [B, L, W] rows for a kernel: a batch of one may come with any, which is not used.
+int64_t batch_stride(const Tensor& t) { return t.size(0) > 1 ? t.stride(0) : t.size(1) * t.size(2); }
+
+bool aligned(const Tensor& t, size_t n) { return (uintptr_t)t.const_data_ptr() % n == 0; }
+
 Tensor bytes(size_t n, const Tensor& like) {
   return at::empty({(int64_t)std::max<size_t>(n, 256)}, like.options().dtype(at::kByte));
 }
@@ -110,7 +115,7 @@ Tensor norm_conv(const Tensor& x, const Tensor& nw, const Tensor& nb, const Tens
                  void* s) {
   const int64_t B = x.size(0), L = x.size(1), D = x.size(2);
   Tensor out = at::empty({B, L, D}, x.options());
-  check("hdcm_norm_conv_fwd", hdcm_norm_conv_fwd(x.const_data_ptr(), x.stride(0), x.stride(1), nw.const_data_ptr(),
+  check("hdcm_norm_conv_fwd", hdcm_norm_conv_fwd(x.const_data_ptr(), batch_stride(x), x.stride(1), nw.const_data_ptr(),
                                                  nb.const_data_ptr(), cw.const_data_ptr(), cb.const_data_ptr(),
                                                  out.mutable_data_ptr(), out.stride(0), out.stride(1), B, L, D,
                                                  (float)eps, dtype_of(x), s));
@@ -128,15 +133,13 @@ std::pair<Tensor, Tensor> norm_conv_bwd(const Tensor& go, const Tensor& x, const
   const size_t n = hdcm_norm_conv_bwd_workspace_bytes(B, L, D);
   Tensor ws = bytes(n, x);
   check("hdcm_norm_conv_bwd_add",
-        hdcm_norm_conv_bwd_add(go.const_data_ptr(), go.stride(0), go.stride(1), x.const_data_ptr(), x.stride(0), x.stride(1),
+        hdcm_norm_conv_bwd_add(go.const_data_ptr(), batch_stride(go), go.stride(1), x.const_data_ptr(), batch_stride(x), x.stride(1),
                            nw.const_data_ptr(), nb.const_data_ptr(), cw.const_data_ptr(), res ? res->const_data_ptr() : nullptr,
                            L * D, D, dx.mutable_data_ptr(),
                            dx.stride(0), dx.stride(1), p, p + D, p + 2 * D, p + 6 * D, ws.mutable_data_ptr(), n, B, L, D,
                            (float)eps, dtype_of(x), s));
   return {dx, dw};
 }
-
-bool aligned(const Tensor& t, size_t n) { return (uintptr_t)t.const_data_ptr() % n == 0; }
 
 // x w^T (+ bias) (+ res) into out, fp32 rows [M, K] and [M, N]
 void gemm_f32(const Tensor& x, const Tensor& w, const float* bias, const float* res, Tensor& out, int64_t M, void* s) {
@@ -288,11 +291,14 @@ Tensor pad_rows(const Tensor& x_, int64_t pad, int64_t stream) {
   const int64_t E = dt == HDCM_BF16 ? 8 : 4;
   Tensor x = x_;
   const int64_t B = x.size(0), L = x.size(1), D = x.size(2);
-  if (x.stride(2) != 1 || x.stride(0) % E || x.stride(1) % E || x.stride(1) < D || (uintptr_t)x.const_data_ptr() % 16)
-    x = x.contiguous();
-  if (D % E || (uintptr_t)x.const_data_ptr() % 16) return at::constant_pad_nd(x, {0, 0, pad, 0});
+  const auto fits = [&] {
+    return x.stride(2) == 1 && (B <= 1 || x.stride(0) % E == 0) && (L <= 1 || (x.stride(1) % E == 0 && x.stride(1) >= D)) &&
+           aligned(x, 16);
+  };
+  if (!fits()) x = x.contiguous();
+  if (D % E || !fits()) return at::constant_pad_nd(x, {0, 0, pad, 0});
   Tensor out = at::empty({B, L + pad, D}, x.options());
-  check("hdcm_pad_rows_fwd", hdcm_pad_rows_fwd(x.const_data_ptr(), x.stride(0), x.stride(1), out.mutable_data_ptr(), B, L,
+  check("hdcm_pad_rows_fwd", hdcm_pad_rows_fwd(x.const_data_ptr(), batch_stride(x), L > 1 ? x.stride(1) : D, out.mutable_data_ptr(), B, L,
                                                pad, D, dt, (void*)stream));
   return out;
 }
@@ -315,8 +321,11 @@ Tensor block_step(const Tensor& x_, const std::vector<Tensor>& params, double ep
   Entry entry;
   on_gpu(x_);
   const Dims d = dims_of(dims);
-  Tensor x = x_.stride(1) == 1 && x_.stride(0) % 8 == 0 && (uintptr_t)x_.const_data_ptr() % 16 == 0 ? x_ : x_.contiguous();
-  const int64_t B = x.size(0), dm = x.size(1), ds = d.ds, hd = dm / d.H, K = ds + dm;
+  TORCH_CHECK(x_.dim() == 2, "step expects x of shape [B, d_model]");
+  const bool fits =
+      x_.stride(1) == 1 && (x_.size(0) <= 1 || x_.stride(0) % (16 / x_.element_size()) == 0) && aligned(x_, 16);
+  const Tensor x = fits ? x_ : x_.clone(at::MemoryFormat::Contiguous);
+  const int64_t B = x.size(0), dm = x.size(1), ds = d.ds, hd = dm / d.H, K = ds + dm, xs = B > 1 ? x.stride(0) : dm;
   const Params p = params_of(params, x, eps);
   const int64_t N = p.w_in.size(0);
   const int dt = dtype_of(x);
@@ -333,14 +342,14 @@ Tensor block_step(const Tensor& x_, const std::vector<Tensor>& params, double ep
   if (fused_front && rows16 && dm % 32 == 0 && dm <= 2048 && N >= 2048) {
     TORCH_CHECK(step_ws, "step: the fused front needs its workspace");
     check("hdcm_norm_conv_in_proj_step_fwd",
-          hdcm_norm_conv_in_proj_step_fwd(x.const_data_ptr(), x.stride(0), p.nw.const_data_ptr(), p.nb.const_data_ptr(),
+          hdcm_norm_conv_in_proj_step_fwd(x.const_data_ptr(), xs, p.nw.const_data_ptr(), p.nb.const_data_ptr(),
                                           p.cw.const_data_ptr(), p.cb.const_data_ptr(), conv.mutable_data_ptr(), (float)eps,
                                           u.mutable_data_ptr(), dm, p.w_in.const_data_ptr(), dm, p.b_in.const_data_ptr(),
                                           projs.mutable_data_ptr(), N, B, dm, N, step_ws->mutable_data_ptr(),
                                           step_ws->numel(), dt, s));
   } else {
     check("hdcm_norm_conv_step_fwd",
-          hdcm_norm_conv_step_fwd(x.const_data_ptr(), x.stride(0), p.nw.const_data_ptr(), p.nb.const_data_ptr(),
+          hdcm_norm_conv_step_fwd(x.const_data_ptr(), xs, p.nw.const_data_ptr(), p.nb.const_data_ptr(),
                                   p.cw.const_data_ptr(), p.cb.const_data_ptr(), conv.mutable_data_ptr(),
                                   u.mutable_data_ptr(), dm, B, dm, (float)eps, dt, s));
     if (bf && B <= 16 && dm % 32 == 0 && dm <= 3072) {
@@ -359,7 +368,7 @@ Tensor block_step(const Tensor& x_, const std::vector<Tensor>& params, double ep
   if (fused_out) {
     Tensor y = at::empty({B, dm}, x.options());
     check("hdcm_rowln_gemm_fwd",
-          hdcm_rowln_gemm_fwd(c.const_data_ptr(), K, p.w_out.const_data_ptr(), K, x.const_data_ptr(), x.stride(0),
+          hdcm_rowln_gemm_fwd(c.const_data_ptr(), K, p.w_out.const_data_ptr(), K, x.const_data_ptr(), xs,
                               y.mutable_data_ptr(), dm, B, dm, K, 1e-5f, dt, s));
     return y;
   }
@@ -368,7 +377,7 @@ Tensor block_step(const Tensor& x_, const std::vector<Tensor>& params, double ep
     Tensor y = at::empty({B, dm}, x.options());
     check("hdcm_skinny_gemm_fwd",
           hdcm_skinny_gemm_fwd(c.const_data_ptr(), K, p.w_out.const_data_ptr(), K, nullptr, x.const_data_ptr(),
-                               x.stride(0), y.mutable_data_ptr(), dm, B, dm, K, dt, s));
+                               xs, y.mutable_data_ptr(), dm, B, dm, K, dt, s));
     return y;
   }
   return at::addmm(x, c, p.w_out.t());
@@ -426,7 +435,8 @@ std::vector<Tensor> mixer_backward(const Tensor& dcomb_, const Tensor& projs, co
                                    const DimArgs& dims, int64_t stream) {
   Entry entry;
   on_gpu(dcomb_);
-  const Tensor dcomb = same(dcomb_, projs, "grad");
+  Tensor dcomb = same(dcomb_, projs, "grad");
+  if (!aligned(dcomb, 16)) dcomb = dcomb.clone();
   const Dims d = dims_of(dims);
   auto g = mixer_grads(projs, same(A_log, projs, "A_log"), same(gamma, projs, "gamma"), same(gnw, projs, "gn_w"),
                        same(gnb, projs, "gn_b"), combined, slot_ws, dcomb, d, (void*)stream);

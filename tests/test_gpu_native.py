@@ -216,6 +216,44 @@ def test_training_gradients_in_the_parameters_types(dev):
         assert not torch.equal(t, t.bfloat16().float())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C", [64, 50])  # without and with padding at 100 rows
+def test_single_sequence_of_any_batch_stride(dev, dtype, C):
+    """A batch of one may come with any batch stride (one sequence of a batch whose sequences are a few
+    values apart), a token row likewise."""
+    _say("batch stride", dtype, C)
+    blk = _block(dev, dtype, C=C).eval()
+    buf = torch.randn(2, 100 * 256 + 3, device=dev).to(dtype)
+    x = buf[:, :100 * 256].view(2, 100, 256)[:1]
+    xc = x.clone(memory_format=torch.contiguous_format)
+    assert x.stride(0) % 4 == 3
+    with torch.no_grad():
+        assert torch.equal(blk(x)[0], blk(xc)[0])
+        a, b = blk.prefill(x), blk.prefill(xc)
+        assert torch.equal(a[0], b[0])
+        assert torch.equal(blk.step(buf[:1, :256], a[1]), blk.step(buf[:1, :256].clone(memory_format=torch.contiguous_format), b[1]))
+    blk.train()
+    g = [torch.autograd.grad(blk(t)[0].sum(), [blk.out_proj.weight])[0] for t in (x, xc)]
+    assert torch.equal(*g)
+
+
+@pytest.mark.parametrize("H,dm", [(4, 192), (4, 256)])
+def test_mixer_gradient_of_an_unaligned_upstream(dev, H, dm):
+    """The mixer's upstream gradient may be contiguous at any address."""
+    from hdcmamba_amd.model import SlotSsmMixerFunction
+
+    _say("unaligned upstream gradient", H, dm)
+    ds = 32
+    projs = (0.5 * torch.randn(1, 64, 3 * ds + 4 * dm, device=dev)).requires_grad_()
+    A = torch.log(torch.linspace(0.5, 2.0, ds, device=dev))
+    out = SlotSsmMixerFunction.apply(projs, A, torch.full((H,), 0.95, device=dev), torch.ones(dm, device=dev),
+                                     torch.zeros(dm, device=dev), ds, dm, H, 64)
+    flat = torch.randn(out.numel() + 1, device=dev)
+    dy = flat[1:].view(out.shape)
+    a, b = (torch.autograd.grad(out, [projs], t, retain_graph=True)[0] for t in (dy, dy.clone()))
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("mixer", [False, True])
 @pytest.mark.parametrize("dtype,region", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float16)])
 def test_training_backward_in_an_autocast_region(dev, mixer, dtype, region):

@@ -405,6 +405,12 @@ _ssm_ws = {}       # (device index, stream) -> the scan's persistent workspace
 _ssm_ws_kept = []  # replaced workspaces stay allocated: a recorded graph may still use them
 
 
+def _ssm_no_capture():
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("ssm: the scan's workspace must exist before graph capture; run the "
+                           "forward once outside capture first")
+
+
 def _ssm_workspace(device, nbytes):
     """The scan's workspace for the current stream of `device`: zero-filled once, then reused
     by every call on that stream (the kernel keeps it consistent; calls on one stream are
@@ -413,9 +419,7 @@ def _ssm_workspace(device, nbytes):
     key = (stream.device.index, stream.cuda_stream)
     ws = _ssm_ws.get(key)
     if ws is None or ws.numel() < nbytes:
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("ssm: the scan's workspace must exist before graph capture; run the "
-                               "forward once outside capture first")
+        _ssm_no_capture()
         if ws is not None:
             _ssm_ws_kept.append(ws)
         ws = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
@@ -433,8 +437,10 @@ def native_streams(t, L, d_state, overlap):
     side = side_stream(t.device)
     ws = _ssm_ws.get((side.device.index, side.cuda_stream))
     if ws is None or ws.numel() < nbytes:
+        _ssm_no_capture()  # (asked of the caller's stream: the side stream would not be capturing)
         with torch.cuda.stream(side):
             ws = _ssm_workspace(t.device, nbytes)
+        main.wait_stream(side)  # a graph recorded from main uses it after the zero fill
     if overlap == "auto":
         if not torch.cuda.is_current_stream_capturing():
             ws = _ssm_workspace(t.device, nbytes)

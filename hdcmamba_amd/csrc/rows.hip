@@ -2,8 +2,6 @@
 // one stream after another.
 #include <math.h>
 
-#include <vector>
-
 #include "hdcm_common.h"
 
 using namespace hdcm;
@@ -40,16 +38,6 @@ __global__ __launch_bounds__(kThreads) void gamma_kernel(const T* __restrict__ d
   gamma[h] = from_f<T>(expf(-sp));
 }
 
-// One event per thread and device: a wait takes the event's state when it is issued, so the event
-// can be recorded again at once.
-hipEvent_t order_event(int device) {
-  static thread_local std::vector<hipEvent_t> events;
-  if (device < 0) return nullptr;
-  if ((size_t)device >= events.size()) events.resize(device + 1, nullptr);
-  if (!events[device] && hipEventCreateWithFlags(&events[device], hipEventDisableTiming) != hipSuccess) events[device] = nullptr;
-  return events[device];
-}
-
 }  // namespace
 
 extern "C" int hdcm_pad_rows_fwd(const void* src, int64_t src_batch_stride, int64_t src_row_stride, void* dst, int64_t B,
@@ -84,10 +72,19 @@ extern "C" int hdcm_gamma_fwd(const void* decay_log, void* gamma, int64_t H, int
   return hdcm_launch_status();
 }
 
+// An event of the call's own, on the streams' device: a wait holds what it needs of the event, which is given
+// back here (nothing is kept per thread, and a captured event is never recorded again outside its capture).
 extern "C" int hdcm_stream_after(void* stream, void* after, int device) {
   if (stream == after) return HDCM_OK;
-  const hipEvent_t e = order_event(device);
-  HDCM_CHECK_ARG(e != nullptr, HDCM_ELAUNCH);
-  if (hipEventRecord(e, (hipStream_t)after) != hipSuccess) return HDCM_ELAUNCH;
-  return hipStreamWaitEvent((hipStream_t)stream, e, 0) == hipSuccess ? HDCM_OK : HDCM_ELAUNCH;
+  HDCM_CHECK_ARG(device >= 0, HDCM_EINVAL);
+  int current = device;
+  if (hipGetDevice(&current) != hipSuccess || (current != device && hipSetDevice(device) != hipSuccess)) return HDCM_ELAUNCH;
+  hipEvent_t e = nullptr;
+  bool ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  if (ok) {
+    ok = hipEventRecord(e, (hipStream_t)after) == hipSuccess && hipStreamWaitEvent((hipStream_t)stream, e, 0) == hipSuccess;
+    (void)hipEventDestroy(e);
+  }
+  if (current != device) (void)hipSetDevice(current);
+  return ok ? HDCM_OK : HDCM_ELAUNCH;
 }

@@ -288,3 +288,40 @@ def test_step_refuses_a_state_elsewhere(dev):
             assert torch.isfinite(blk.step(x[:, 0], st)).all(), path
         with pytest.raises(RuntimeError, match="cpu"):
             blk.step(x[:, 0], st, pos_dev=torch.zeros(1, dtype=torch.int32))
+
+
+def test_scan_overlap_from_threads_and_in_a_graph(dev):
+    """The scan on the side stream gives the same rows from short-lived threads and from every replay of a
+    recorded forward, with eager forwards between the replays."""
+    import threading
+
+    _say("overlap threads, graph")
+    blk = _block(dev, torch.bfloat16).eval()
+    x = _x(dev, 128, torch.bfloat16)
+    with torch.no_grad():
+        want = blk(x)[0]
+        other = blk(-x)[0]
+    for mode in ("none", "state", "gate", "after_state"):
+        blk.ssm_overlap = mode
+        got = []
+
+        def work():
+            with torch.no_grad():
+                got.append(blk(x)[0])
+
+        for _ in range(3):
+            t = threading.Thread(target=work)
+            t.start()
+            t.join()
+        assert len(got) == 3 and all(torch.equal(g, want) for g in got), mode
+        xs = x.clone()
+        with torch.no_grad():
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                y = blk(xs)[0]
+            for k in range(4):
+                xs.copy_(x if k % 2 else -x)
+                graph.replay()
+                assert torch.equal(blk(x)[0], want), (mode, k)
+                torch.cuda.synchronize()
+                assert torch.equal(y, want if k % 2 else other), (mode, k)

@@ -325,3 +325,43 @@ def test_scan_overlap_from_threads_and_in_a_graph(dev):
                 assert torch.equal(blk(x)[0], want), (mode, k)
                 torch.cuda.synchronize()
                 assert torch.equal(y, want if k % 2 else other), (mode, k)
+
+
+def test_training_on_two_streams(dev):
+    """Two blocks trained from two threads, each on a stream of its own, get the gradients of one after the
+    other: nothing but the weights' own storage is shared."""
+    import threading
+
+    _say("two streams")
+    blocks = [_block(dev, torch.bfloat16, mixer=True, seed=s) for s in (3, 4)]
+    xs = [_x(dev, L, torch.bfloat16, seed=L) for L in (1000, 700)]
+
+    def step(i):
+        blk, x = blocks[i], xs[i]
+        y = blk(x)[0]
+        return torch.autograd.grad(y, [blk.out_proj.weight, blk.in_proj.weight, blk.A_log], torch.ones_like(y))
+
+    want = [step(i) for i in range(2)]
+    torch.cuda.synchronize()
+    got, errors = [[], []], []
+    gate = threading.Barrier(2, timeout=60)
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream(dev)):
+                step(i)
+                gate.wait()
+                got[i] = [step(i) for _ in range(8)]
+                torch.cuda.current_stream(dev).synchronize()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for i in range(2):
+        for g in got[i]:
+            assert all(torch.equal(a, b) for a, b in zip(g, want[i])), i

@@ -98,15 +98,24 @@ struct Params {
   Tensor nw, nb, cw, cb, w_in, b_in, A_log, gamma, gnw, gnb, w_out;
   double eps;
 };
-Params params_of(const std::vector<Tensor>& p, const Tensor& x, double eps) {
+Params params_of(const std::vector<Tensor>& p, const Tensor& x, const Dims& d, double eps) {
   TORCH_CHECK(p.size() == 11, "a block has 11 parameters");
-  const int64_t dm = x.size(-1);
+  const int64_t dm = x.size(-1), K = d.ds + dm;
   static const char* names[] = {"norm.weight", "norm.bias", "conv1d.weight", "conv1d.bias", "in_proj.weight",
                                 "in_proj.bias", "A_log", "gamma_buf", "group_norm.weight", "group_norm.bias",
                                 "out_proj.weight"};
   std::vector<Tensor> q;
   q.reserve(11);
   for (size_t i = 0; i < 11; ++i) q.push_back(same(p[i], x, names[i]));
+  // the kernels get pointers: the projections' shapes as a product would check them, the vectors' lengths
+  const Tensor &w_in = q[4], &w_out = q[10];
+  TORCH_CHECK(w_in.dim() == 2 && w_in.size(1) == dm && w_in.size(0) >= 3 * d.ds + 4 * dm && q[5].numel() == w_in.size(0),
+              "in_proj ", w_in.sizes(), " + ", q[5].sizes(), " does not take x of width ", dm);
+  TORCH_CHECK(w_out.dim() == 2 && w_out.size(1) == K && w_out.size(0) == dm, "out_proj ", w_out.sizes(), " should be [", dm, ", ",
+              K, "]");
+  const int64_t least[] = {dm, dm, 4 * dm, dm, 0, 0, d.ds, d.H, dm, dm};
+  for (size_t i = 0; i < 10; ++i)
+    TORCH_CHECK(q[i].numel() >= least[i], names[i], " has ", q[i].numel(), " values, expected ", least[i]);
   return {q[0], q[1], q[2].view({dm, 4}), q[3], q[4], q[5], q[6], q[7], q[8], q[9], q[10], eps};
 }
 
@@ -278,7 +287,7 @@ Tensor block_forward(const Tensor& x, const std::vector<Tensor>& params, double 
   on_gpu(x);
   const Dims d = dims_of(dims);
   const int64_t B = x.size(0), dm = x.size(2), hd = dm / d.H;
-  return forward(x, params_of(params, x, eps), d, streams_of(streams), out, fused, w_sums, library,
+  return forward(x, params_of(params, x, d, eps), d, streams_of(streams), out, fused, w_sums, library,
                  opt_ptr(h_final, {B, d.ds}, x, "h"), opt_ptr(S_final, {B, d.H, hd, hd}, x, "S_prev"))
       .y;
 }
@@ -326,7 +335,7 @@ Tensor block_step(const Tensor& x_, const std::vector<Tensor>& params, double ep
       x_.stride(1) == 1 && (x_.size(0) <= 1 || x_.stride(0) % (16 / x_.element_size()) == 0) && aligned(x_, 16);
   const Tensor x = fits ? x_ : x_.clone(at::MemoryFormat::Contiguous);
   const int64_t B = x.size(0), dm = x.size(1), ds = d.ds, hd = dm / d.H, K = ds + dm, xs = B > 1 ? x.stride(0) : dm;
-  const Params p = params_of(params, x, eps);
+  const Params p = params_of(params, x, d, eps);
   const int64_t N = p.w_in.size(0);
   const int dt = dtype_of(x);
   void* s = (void*)stream;
@@ -497,7 +506,7 @@ std::vector<OptTensor> block_backward(const Tensor& x, const Tensor& dy, const s
   on_gpu(x);
   const Dims d = dims_of(dims);
   const Streams st = streams_of(streams);
-  const Params p = params_of(params, x, eps);
+  const Params p = params_of(params, x, d, eps);
   const int64_t B = x.size(0), L = x.size(1), dm = x.size(2), M = B * L, K = d.ds + dm, N = p.w_in.size(0);
   std::vector<OptTensor> out(12);
   const auto give = [&](int i, const Tensor& g) {  // i: params_of's index

@@ -365,3 +365,29 @@ def test_training_on_two_streams(dev):
     for i in range(2):
         for g in got[i]:
             assert all(torch.equal(a, b) for a, b in zip(g, want[i])), i
+
+
+def test_parameters_of_another_shape_are_refused(dev):
+    """A projection that does not fit x, or a parameter that is too short, is an error before any launch."""
+    _say("parameter shapes")
+    blk = _block(dev, mixer=True)
+    x = _x(dev, 64)
+    ds, dm, N = 64, 256, 3 * 64 + 4 * 256
+    swaps = [("in_proj", torch.nn.Linear(dm + 8, N)), ("in_proj", torch.nn.Linear(dm - 8, N)),
+             ("out_proj", torch.nn.Linear(dm, dm, bias=False)), ("out_proj", torch.nn.Linear(ds + dm, dm - 8, bias=False)),
+             ("group_norm", torch.nn.GroupNorm(4, dm - 64)), ("norm", torch.nn.LayerNorm(dm - 64))]
+    for name, layer in swaps:
+        kept = getattr(blk, name)
+        setattr(blk, name, layer.to(dev))
+        with pytest.raises(RuntimeError):
+            blk(x)
+        with torch.no_grad(), pytest.raises(RuntimeError):
+            blk(x)
+        with torch.no_grad(), pytest.raises(RuntimeError):
+            blk.step(x[:, 0], blk.new_state(2, dev, x.dtype))
+        setattr(blk, name, kept)
+    blk.A_log.data = blk.A_log.data[:-1]
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        blk(x)
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        blk.step(x, blk.new_state(2, dev, x.dtype))  # (a token row has two dimensions)

@@ -411,9 +411,8 @@ class HdcMamba9v3Block(nn.Module):
         the composition runs with autograd, the row LayerNorm in a pass of its own before out_proj
         (two-pass variance, the weight as it is now: the folded form reads row sums kept until the
         weight's version changes, which a write through ``.data`` or a flat buffer does not do)."""
-        w = self.out_proj.weight
         fused = not train and self._fused_out(x)
-        sums = self._out_weight_sums(w.to(x.dtype)) if fused and _ops.rowln_stats_ok(x, self.d_model) else None
+        sums = self._out_weight_sums(x.dtype) if fused and _ops.rowln_stats_ok(x, self.d_model) else None
         return _ops.native().block_forward(
             x, self._params(), self.norm.eps, (self.d_state, self.num_heads, self.chunk_size), self._native_streams(x),
             out, fused, sums, torch.cuda.tunable.is_enabled(), None if state is None else state.h,
@@ -439,18 +438,18 @@ class HdcMamba9v3Block(nn.Module):
         tiles = -(-rows // 256) * -(-self.d_model // 256)
         return rows <= 16 or tiles <= 1024
 
-    def _out_weight_sums(self, w):
-        """Row sums of the out_proj weight as used (``w``, the activation-dtype weight), kept
-        until the parameter changes (its storage or its version counter).  A refresh writes
-        into the same buffer, so a recorded graph that reads it sees the new sums."""
+    def _out_weight_sums(self, dtype):
+        """Row sums of the out_proj weight as used (in ``dtype``), kept until the parameter changes (its
+        storage or its version counter).  A refresh writes into the same buffer, so a recorded graph
+        that reads it sees the new sums."""
         p = self.out_proj.weight
-        key = (p.data_ptr(), p._version, w.dtype, w.device)
+        key = (p.data_ptr(), p._version, dtype, p.device)
         if getattr(self, "_wsum_key", None) != key:
             old = getattr(self, "_wsum", None)
-            if old is not None and old.device == w.device and old.numel() == w.shape[0]:
-                _ops.row_sums(w, out=old)
+            if old is not None and old.device == p.device and old.numel() == p.shape[0]:
+                _ops.row_sums(p.to(dtype), out=old)
             else:
-                self._wsum = _ops.row_sums(w)
+                self._wsum = _ops.row_sums(p.to(dtype))
             self._wsum_key = key
         return self._wsum
 
@@ -462,7 +461,7 @@ class HdcMamba9v3Block(nn.Module):
             return
         p = self.out_proj.weight
         if (p.data_ptr(), p._version) != self._wsum_key[:2]:
-            self._out_weight_sums(p.to(self._wsum_key[2]))
+            self._out_weight_sums(self._wsum_key[2])
 
     def _fused_mixer_out(self, x, state, out=None):
         """x + out_proj(LN(combined)) for the fused path, x [B,L,dm]; into ``out`` (which may be
@@ -477,7 +476,7 @@ class HdcMamba9v3Block(nn.Module):
             parts = _ops.ssm_stats_parts(self.d_state) + self.num_heads
             stats = torch.empty(parts, B * L, 2, device=x.device, dtype=torch.float32)
             c = self._mixer(x, state, normalize=False, row_stats=stats)
-            y = _ops.rowln_gemm_stats(c, w, self._out_weight_sums(w), stats, x2, out=o2)
+            y = _ops.rowln_gemm_stats(c, w, self._out_weight_sums(w.dtype), stats, x2, out=o2)
         else:
             c = self._mixer(x, state, normalize=False)
             y = _ops.rowln_gemm(c, w, x2, out=o2)

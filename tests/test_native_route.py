@@ -28,3 +28,26 @@ def test_native_path_rule(monkeypatch):
         assert not blk._native_ok(x)
     blk.ssm_overlap = "unknown"
     assert not blk._native_ok(x)
+
+
+def test_out_proj_row_sums_are_formed_once(monkeypatch):
+    """The kept row sums of out_proj's weight in another type: the weight is cast when they are formed, not
+    at every forward, and they follow the weight's version and storage into the same buffer."""
+    blk = HdcMamba9v3Block(64, 8, 2, 8)
+    casts = []
+
+    def row_sums(w, out=None):
+        casts.append(w.dtype)
+        s = w.detach().float().sum(1)
+        return s if out is None else out.copy_(s)
+
+    monkeypatch.setattr(_ops, "row_sums", row_sums)
+    with torch.no_grad():
+        a = blk._out_weight_sums(torch.bfloat16)
+        assert blk._out_weight_sums(torch.bfloat16) is a and casts == [torch.bfloat16]
+        blk.out_proj.weight.add_(1.0)
+        before = a.clone()
+        blk.refresh_derived_weights()
+        blk.refresh_derived_weights()
+        assert len(casts) == 2 and blk._out_weight_sums(torch.bfloat16) is a
+        assert ((a - before) / 72 - 1).abs().max() < 0.01

@@ -589,28 +589,6 @@ def slot_state(projs, q_col, gamma, d_model, num_heads, chunk, ws, S0=None):
     return ws
 
 
-def slot_grad(projs, q_col, gamma, gn_w, gn_b, gn_eps, ws_fwd, dout, dprojs, d_model, num_heads, chunk):
-    """Gradient of slot_state + slot_gate: the q, k, v and gate blocks of dprojs (in place) from
-    dout [B,L,dm] and the forward's workspace ``ws_fwd``; returns (d gn_w, d gn_b) fp32."""
-    _on_gpu(projs, dout, dprojs)
-    B, L, _ = projs.shape
-    if dout.dtype != projs.dtype or dprojs.dtype != projs.dtype or dprojs.shape != projs.shape or dout.shape != (B, L, d_model):
-        raise RuntimeError("slot_grad: dout [B,L,dm] and dprojs must match projs")
-    gamma, gn_w, gn_b = _same(gamma, projs, "gamma"), _same(gn_w, projs, "gn_w"), _same(gn_b, projs, "gn_b")
-    f32 = dict(device=projs.device, dtype=torch.float32)
-    dgw, dgb = torch.empty(d_model, **f32), torch.empty(d_model, **f32)
-    nbytes = lib().hdcm_slot_grad_workspace_bytes(B, L, d_model, num_heads, chunk, _dtype(projs))
-    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=projs.device)
-    ev = timer.begin("slot_grad")
-    _check("hdcm_slot_grad", lib().hdcm_slot_grad(
-        projs.data_ptr(), _rows2d(projs, "projs"), q_col, gamma.data_ptr(), gn_w.data_ptr(), gn_b.data_ptr(),
-        float(gn_eps), ws_fwd.data_ptr(), ws_fwd.numel(), dout.data_ptr(), _rows2d(dout, "dout"), dprojs.data_ptr(),
-        _rows2d(dprojs, "dprojs"), dgw.data_ptr(), dgb.data_ptr(), ws.data_ptr(), ws.numel(), B, L, d_model, num_heads,
-        chunk, _dtype(projs), _stream(projs)))
-    timer.end("slot_grad", ev)
-    return dgw, dgb
-
-
 def slot_attend(base, q_col, k_col, v_col, gamma, d_model, num_heads, chunk, phi, out, out_col, reverse=False,
                 ws=None, chain=None):
     """Slot recurrence without GroupNorm/gate on column blocks of base [B,L,W] into

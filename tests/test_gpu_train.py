@@ -332,3 +332,45 @@ def test_slot_gradient_passes(dev, dtype, B, L, H, hd, ds, C, seg):
 def test_slot_gradient_segments_within_chunks(dev, dtype, B, L, H, hd, ds, C, seg):
     """The same gradients with segments that divide a chunk, in both directions."""
     test_slot_gradient_passes(dev, dtype, B, L, H, hd, ds, C, seg)
+
+
+@pytest.mark.parametrize("dtype,B,L,H,hd,C", [(torch.float32, 2, 192, 2, 64, 64), (torch.bfloat16, 1, 512, 2, 64, 256),
+                                              (torch.bfloat16, 2, 300, 2, 48, 100)])
+def test_slot_gradient_operators(dev, dtype, B, L, H, hd, C):
+    """The slot gradient out of the single operators (y by slot_attend, the GroupNorm and gate backward,
+    the feature maps staged, three attention passes with signed strides and the chain rule in the store
+    or as a pass of its own) against SlotSsmMixerFunction's two passes: fp32 sums in another order;
+    bf16 y and products rounded once more, ~2^-8 of the largest value each."""
+    from hdcmamba_amd import _ops
+    from hdcmamba_amd.model import SlotSsmMixerFunction
+
+    ds, dm = 8, H * hd
+    _say("slot gradient operators", dtype, B, L, H, hd, C)
+    g = torch.Generator(device=dev).manual_seed(L + hd)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    projs, do = rnd(B, L, 3 * ds + 4 * dm).to(dtype), rnd(B, L, ds + dm).to(dtype)
+    gamma, w, b = (0.9 + 0.05 * torch.rand(H, generator=g, device=dev)).to(dtype), (1 + 0.2 * rnd(dm)).to(dtype), (0.1 * rnd(dm)).to(dtype)
+    A_log = torch.log(torch.linspace(0.5, 2.0, ds, device=dev)).to(dtype)
+    leaves = [t.clone().requires_grad_() for t in (projs, w, b)]
+    out = SlotSsmMixerFunction.apply(leaves[0], A_log, gamma, leaves[1], leaves[2], ds, dm, H, C)
+    ref = torch.autograd.grad(out, leaves, do)
+
+    q, gate = 3 * ds, 3 * ds + 3 * dm
+    d = torch.zeros_like(projs)
+    y, z = torch.empty(B, L, dm, device=dev, dtype=dtype), torch.empty(B, L, 4 * dm, device=dev, dtype=dtype)
+    _ops.slot_attend(projs, q, q + dm, q + 2 * dm, gamma, dm, H, C, True, y, 0)
+    dgw, dgb = _ops.gnorm_gate_bwd(y, projs[..., gate:], w, b, 1e-5, do[..., ds:], H, z[..., :dm], d[..., gate:])
+    _ops.slot_phi_prep(projs, q, dm, z)  # z = [dy | v | phi(k) | phi(q)]
+    _ops.slot_attend(z, 2 * dm, 3 * dm, 0, gamma, dm, H, C, False, d, q + 2 * dm, reverse=True)
+    apart = d.clone()
+    _ops.slot_attend(z, 0, dm, 2 * dm, gamma, dm, H, C, False, d, q, chain=projs)
+    _ops.slot_attend(z, dm, 0, 3 * dm, gamma, dm, H, C, False, d, q + dm, reverse=True, chain=projs)
+    _ops.slot_attend(z, 0, dm, 2 * dm, gamma, dm, H, C, False, apart, q)
+    _ops.slot_attend(z, dm, 0, 3 * dm, gamma, dm, H, C, False, apart, q + dm, reverse=True)
+    _ops.slot_phi_chain(projs, q, dm, apart)
+    lim = 1e-4 if dtype == torch.float32 else 2e-2
+    for i, name in enumerate(("d q", "d k", "d v", "d gate")):
+        cols = slice(q + i * dm, q + (i + 1) * dm)
+        for got in (d, apart):
+            assert max_rel(got[..., cols], ref[0][..., cols]) <= lim, name
+    assert max_rel(dgw, ref[1]) <= lim and max_rel(dgb, ref[2]) <= lim

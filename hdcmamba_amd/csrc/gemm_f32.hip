@@ -160,11 +160,15 @@ void launch_tile(const float* x, int64_t x_rs, const float* w, int64_t w_rs, con
 
 }  // namespace
 
-// Up to M N K of 4e10 and K of 1536: beyond, the library's wider tiles are as fast or faster (4096 x 8576 x 2048
-// 1016 against 1076 us, 4096 x 2048 x 2176 264 against 276, 16384 x 4480 x 1024 1090 against 1123).  A few
-// rows (decode steps) stay with it too: 16 x 8576 x 2048 is 21 us against 29.
+// Up to M N K of 4e10 and K of 1152 (d_model 1024's projections).  Beyond that many products the library is
+// as fast (M x N x K, us, library and this: 16384 x 3264 x 768 607, 628; 16384 x 4480 x 1024 1103, 1133).  At
+// wider K it wins below 2048 rows and gives away little above: 64 x 6336 x 1536 18.5, 22.8; 256 rows 50, 56; 512 x
+// 1408 x 1472 25, 33; 512 x 1280 x 1344 22, 30; 1536 x 5312 x 1280 155, 165; 4096 x 6336 x 1536 618, 609.  Within
+// the line its time is uneven, and single sizes lie behind it (128 x 4480 x 1024 19, 23; 384 rows 32, 38; 512 x
+// 3264 x 768 28, 30) among neighbours ahead (256 rows 35, 31; 1000 x 3264 x 768 64, 56).  A few rows (decode
+// steps) stay with it too: 16 x 8576 x 2048 is 21 us against 29.
 extern "C" int hdcm_gemm_f32_preferred(int64_t M, int64_t N, int64_t K) {
-  return M >= 64 && N > 0 && N % 4 == 0 && K > 0 && K <= 1536 && K % 4 == 0 && M <= (int64_t)40000000000 / K / N;
+  return M >= 64 && N > 0 && N % 4 == 0 && K > 0 && K <= 1152 && K % 4 == 0 && M <= (int64_t)40000000000 / K / N;
 }
 
 extern "C" int hdcm_gemm_f32_fwd(const float* x, int64_t x_row_stride, const float* w, int64_t w_row_stride,

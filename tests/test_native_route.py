@@ -51,3 +51,14 @@ def test_out_proj_row_sums_are_formed_once(monkeypatch):
         blk.refresh_derived_weights()
         assert len(casts) == 2 and blk._out_weight_sums(torch.bfloat16) is a
         assert ((a - before) / 72 - 1).abs().max() < 0.01
+
+
+def test_product_rules_at_their_lines():
+    """Which products run on the kernels here: both sides of every line of the rules."""
+    lib = _ops.lib()
+    f32 = lib.hdcm_gemm_f32_preferred
+    assert f32(64, 4480, 1024) and f32(8192, 4480, 1024) and f32(1000, 1024, 1152) and not f32(63, 4480, 1024)
+    assert not f32(16384, 4480, 1024) and not f32(512, 1408, 1472) and not f32(256, 6336, 1536)
+    bf = lambda M, N, K: lib.hdcm_gemm_preferred(M, N, K, _ops.HDCM_BF16)  # noqa: E731
+    assert bf(32768, 3264, 768) and not bf(32769, 3264, 768) and bf(16384, 4480, 1024) and not bf(16385, 4480, 1024)
+    assert not bf(8192, 6336, 1536) and not bf(0, 3264, 768) and not lib.hdcm_gemm_preferred(8192, 3264, 768, 0)

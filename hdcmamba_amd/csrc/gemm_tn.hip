@@ -258,10 +258,16 @@ bool fits32(int64_t rs) { return rs <= ((int64_t)1 << 30) / (2 * kStep); }
 }  // namespace
 
 // From 4096 rows on, 1024 where the column sums are wanted too: the library's product is faster below
-// (2048 x 768 x 832 20 against 23 us), but not with its column-sum kernel (2048 x 2240 x 512 42 against 25).
+// (2048 x 768 x 832 18 against 22 us), but not with its column-sum kernel (2048 x 2240 x 512 40 against 24).
+// Between 4096 and 10240 rows the library keeps outputs of 8 to 20 million values (in_proj at d_model 1536 and
+// 2048), whose split leaves this kernel two partial rounds (rows x N x K, library and this: 4096 x 6336 x 1536
+// 105, 124; 8192 185, 195; 10240 227, 242; 4096 x 8576 x 2048 184, 197; 8192 340, 374); the lines lie where the two
+// cross: 3000 x 6336 x 1536 92, 92; 12288 379, 285; 8192 x 5184 x 1280 144, 133; 8192 x 10624 x 2560 578, 533.
 extern "C" int hdcm_gemm_tn_preferred(int64_t M, int64_t N, int64_t K, int col_sums, int dtype) {
-  return dtype == HDCM_BF16 && M >= (col_sums ? 1024 : 4096) && N % 8 == 0 && K % 8 == 0 && N > 0 && K > 0 &&
-         M < (int64_t)1 << 30 && N < (int64_t)1 << 24 && K < (int64_t)1 << 24 && fits32(N) && fits32(K);
+  if (!(dtype == HDCM_BF16 && M >= (col_sums ? 1024 : 4096) && N % 8 == 0 && K % 8 == 0 && N > 0 && K > 0 &&
+        M < (int64_t)1 << 30 && N < (int64_t)1 << 24 && K < (int64_t)1 << 24 && fits32(N) && fits32(K)))
+    return 0;
+  return !(M >= 4096 && M <= 10240 && N * K >= 8000000 && N * K <= 20000000);
 }
 
 extern "C" size_t hdcm_gemm_tn_workspace_bytes(int64_t M, int64_t N, int64_t K) {

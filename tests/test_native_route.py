@@ -59,6 +59,11 @@ def test_product_rules_at_their_lines():
     f32 = lib.hdcm_gemm_f32_preferred
     assert f32(64, 4480, 1024) and f32(8192, 4480, 1024) and f32(1000, 1024, 1152) and not f32(63, 4480, 1024)
     assert not f32(16384, 4480, 1024) and not f32(512, 1408, 1472) and not f32(256, 6336, 1536)
+    tn = lambda M, N, K, sums: lib.hdcm_gemm_tn_preferred(M, N, K, sums, _ops.HDCM_BF16)  # noqa: E731
+    assert tn(1024, 2240, 512, 1) and not tn(1023, 2240, 512, 1) and tn(4096, 768, 832, 0) and not tn(4095, 768, 832, 0)
+    for N, K in ((6336, 1536), (8576, 2048)):  # one partial round of split tiles more than the library
+        assert tn(4095, N, K, 1) and not tn(4096, N, K, 1) and not tn(10240, N, K, 1) and tn(10241, N, K, 1)
+    assert tn(8192, 5184, 1280, 1) and tn(8192, 10624, 2560, 1)
     bf = lambda M, N, K: lib.hdcm_gemm_preferred(M, N, K, _ops.HDCM_BF16)  # noqa: E731
     assert bf(32768, 3264, 768) and not bf(32769, 3264, 768) and bf(16384, 4480, 1024) and not bf(16385, 4480, 1024)
     assert not bf(8192, 6336, 1536) and not bf(0, 3264, 768) and not lib.hdcm_gemm_preferred(8192, 3264, 768, 0)

@@ -557,9 +557,12 @@ extern "C" int hdcm_gemm_fwd(const void* x, int64_t x_row_stride, const void* w,
 }
 
 // Where the library's default solution measured slower (in_proj, N = 4 K + 192 or 4 K + 384; us, library and
-// this): K 768, 32768 rows 265, 171; 8192 rows 70, 49; K 256, 16384 rows 34, 24; K 1024, 16384 rows
-// 161, 150; 1024 rows 19.2, 18.6.  Beyond it is as fast or faster: K 768, 65536 rows 314, 336; K 1024,
-// 32768 rows 251, 273; K 512, 131072 rows 376, 397; K 1536, 8192 rows 154, 161; K 2048, 16128 rows 419, 469.
+// this): K 768, 32768 rows 265, 171 (N 3456 166, 171); 8192 rows 70, 49; K 256, 16384 rows 34, 24; K 1024,
+// 16384 rows 161, 150; 1024 rows 19.2, 18.6.  Above 32768 rows its time jumps between neighbours and the
+// line is on the safe side (K 768: 36864 rows 199, 194; 40960 329, 218; 49152 291, 242; 57344 291, 287; 65536
+// 316, 338; N 3456: 36864 rows 189, 196; 57344 449, 318; 65536 328, 362; K 512: 36864 rows 149, 108; 65536
+// 206, 169; 131072 376, 397).  K 1024: 28672 rows 227, 242; 32768 251, 275 (N 4288 285, 271); 49152 414, 418.
+// K 1536, 8192 rows 154, 161; K 2048, 16128 rows 419, 469.
 extern "C" int hdcm_gemm_preferred(int64_t M, int64_t N, int64_t K, int dtype) {
   return dtype == HDCM_BF16 && K > 0 && K <= 1024 && K % 8 == 0 && N > 0 && N % 4 == 0 && M > 0 &&
          M <= (K <= 768 ? 32768 : 16384);

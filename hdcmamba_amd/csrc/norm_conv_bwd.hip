@@ -376,9 +376,10 @@ int launch_bwd(const void* go, int64_t g_bs, int64_t g_rs, const void* x, int64_
 
 extern "C" size_t hdcm_norm_conv_bwd_workspace_bytes(int64_t B, int64_t L, int64_t D) {
   if (B <= 0 || L <= 0 || D <= 0) return 0;
-  // the size this entry point has always asked for, which covers the sums at most shapes
-  const size_t asked = (size_t)((B * L * sizeof(float2) + 255) / 256) * 256 + (size_t)B * ((L + 63) / 64) * 7 * D * sizeof(float);
-  return std::max(asked, (size_t)plan_of(B, L, D).grid * 5 * D * sizeof(float));
+  // The size callers lay out (8 bytes a row and 7 D floats per 64 rows), kept so that a buffer of it stays
+  // enough; the sums take 5 D floats per workgroup, more than that only at many short sequences.
+  const size_t laid_out = (size_t)((B * L * sizeof(float2) + 255) / 256) * 256 + (size_t)B * ((L + 63) / 64) * 7 * D * sizeof(float);
+  return std::max(laid_out, (size_t)plan_of(B, L, D).grid * 5 * D * sizeof(float));
 }
 
 extern "C" int hdcm_norm_conv_bwd_add(const void* grad_out, int64_t g_batch_stride, int64_t g_row_stride,

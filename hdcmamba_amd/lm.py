@@ -162,8 +162,7 @@ class ForwardGraph:
     A forward at B=1, L=32768 issues about 170 kernels (seven per block); launched one by
     one from Python they leave the GPU idle between launches (eager forwards ~15.6 ms against
     ~14.2 ms replayed).
-    A replay submits the recorded sequence at once, including the side-stream fork and
-    join of every block.  ``forward(input_ids)`` copies the ids into the static input
+    A replay submits the recorded sequence at once.  ``forward(input_ids)`` copies the ids into the static input
     buffer and returns the static logits buffer, which the next replay overwrites.  The
     weights are read at replay time (in place updates are seen: values derived from a
     weight and kept between forwards, the out_proj row sums, are refreshed in place before

@@ -1,7 +1,8 @@
 """hipBLASLt solution selection for the block's GEMMs (in_proj, out_proj, tied LM head).
 
-The projections stay library GEMMs; what this module changes is which hipBLASLt solution
-runs them.  PyTorch's TunableOp benchmarks every hipBLASLt/rocBLAS solution for a GEMM
+With recorded solutions in use the projections of the forward are library GEMMs throughout (without
+them some sizes run on this package's own); what this module changes is which hipBLASLt
+solution runs them.  PyTorch's TunableOp benchmarks every hipBLASLt/rocBLAS solution for a GEMM
 signature (transposes, M, N, K, leading dimensions, bias) and records the fastest in a CSV
 file whose header pins the PyTorch, HIP, hipBLASLt and rocBLAS versions and the GPU
 architecture.  ``use_tuned_gemms()`` loads the file shipped beside this module with tuning

@@ -159,10 +159,10 @@ class ForwardGraph:
     """The inference forward of an HdcMambaLM at one input shape, recorded once as a HIP
     graph and replayed per call.
 
-    A forward at B=1, L=32768 issues about 170 kernels (seven per block); launched one by
-    one from Python they leave the GPU idle between launches (eager forwards ~15.6 ms against
-    ~14.2 ms replayed).
-    A replay submits the recorded sequence at once.  ``forward(input_ids)`` copies the ids into the static input
+    A forward at B=1, L=32768 issues about 170 kernels (seven per block).  A replay submits the
+    recorded sequence at once: the same time as an eager forward there (14.3 ms both; one native
+    call per block keeps ahead of the GPU), less where the kernels are short.
+    ``forward(input_ids)`` copies the ids into the static input
     buffer and returns the static logits buffer, which the next replay overwrites.  The
     weights are read at replay time (in place updates are seen: values derived from a
     weight and kept between forwards, the out_proj row sums, are refreshed in place before
